@@ -450,16 +450,6 @@ struct NoProps {
     __device__ void publish() const {}
 };
 
-// Compensated FP32 accumulation (Knuth's TwoSum): s + c carries the sum of
-// the added values with an error of O(u^2) relative to their magnitudes.
-__device__ __forceinline__ void two_sum_add(float& s, float& c, float x) {
-    const float t = s + x;
-    const float bp = t - s;
-    const float e = (s - (t - bp)) + (x - bp);
-    s = t;
-    c += e;
-}
-
 // ---- wavefront helpers (64 lanes) ---------------------------------------
 
 __device__ __forceinline__ int lane_id() { return __lane_id(); }

@@ -17,60 +17,121 @@
 //   - Markers arrive sorted by fine key (ereb_sort.hip): a tile's markers are
 //     contiguous and grouped by fine cell in ascending marker index.
 //
-// One workgroup per tile (eight wavefronts in the Float64 form, four in the
-// mixed form; ScatterShape below).  The tile is walked one basic
-// column at a time: the column's 24 fine cells (fine columns 2k, 2k+1) hold a
-// contiguous run of sorted markers, split into chunks of at most CH markers
-// when it is longer.  Per chunk, between two workgroup barriers:
-//   1. tasks  : wavefronts g and g + 4 own the first and second half of the
-//               sums of grid g (basic, Vx, Vy, P; the second half includes
-//               the weight sum); with four wavefronts, wavefront g owns them
-//               all.  A task is (fine cell, corner column cj): the sums over
-//               the fine cell's markers, in order, of property * weight for
-//               the corners (0, cj) and (1, cj), and of the weights;
-//   2. combine: lane (r, c) of a wavefront owns window node (r, c) of its
-//               grid and adds the partials of the at most 8 fine cells of the
-//               column that touch it, in a fixed (column, fine column, fine
-//               row) order; then
-//      stage  : the next chunk's markers (two threads per marker, one per
-//               half of its inputs; one thread in the four-wavefront form)
-//               stage their 18 property values and the fractions dxmj/dx,
-//               dymi/dy of the basic and P stencils in LDS.  Their inputs
-//               were loaded into registers before step 1, so the gather
-//               latency overlaps steps 1 and 2, and the staging overlaps
-//               other wavefronts' combine.
+// One workgroup per tile.  The sums of one fine cell are a contraction over
+// its markers: (corner weights)^T x (property values), 4 corners by up to 10
+// values for each of the four grids.  They run on the FP64 matrix cores
+// (v_mfma_f64_4x4x4_4b: four independent 4x4x4 products an instruction, each
+// element the chain of fmas over its k in ascending order): the four blocks b
+// are four fine cells, k four markers of a block's fine cell, the rows the four
+// corners and the columns four property values.
+//   Lane l of the operands: t = l & 3, block b = l >> 2 & 3, k = l >> 4 (A row
+// t, B column t); lane l of the result: column l & 3, block l >> 2 & 3, row
+// l >> 4.
+//   The four blocks are four fine cells on top of each other, whose markers are
+// one run of the sort order; a wavefront walks its four fine rows across a
+// segment of fine columns, its markers in groups of up to four a block (a fine
+// column has as many groups as its fullest cell needs).  A chunk is four
+// consecutive groups, of one fine column or of several: lane t of a quad loads
+// the values of its block's k-th marker of group t (neighbouring lanes take
+// neighbouring markers, so a load's lanes read the few cache lines of the
+// cells' marker columns), a 4x4 transpose inside each quad of lanes turns them
+// into the products' B operands (no marker value goes through LDS), and the
+// marker's four stencil fractions reach the A operands by quad broadcasts.  The
+// next chunk's values are loaded before this chunk's products, the marker
+// numbers of the one after that too; no barrier separates the chunks.
+//   The blocks lie on top of each other because a cache line holds 16 markers of
+// one marker column: with the blocks side by side, walking down, every line was
+// fetched five times (15 against 3.5 million L2 requests at 2.8M markers, 215
+// against 150 us).  Staging the values in LDS with the sums in vector
+// instructions, two barriers a chunk, took 173 us (2.8M markers, Float64; mixed
+// form 131) and 1,426 us (20M, 16 markers a fine cell); this takes 134 (110) and
+// 604 us, 3.5 TB/s of the 160 algorithmic bytes a marker at 2.8M.  What bounds
+// it: about half vector and matrix issue (timed with the loads left out 98 us),
+// half the loads' latency, three wavefronts a SIMD (five in the mixed form).
+//   Row q of A and of the result: node column parity q >> 1, node row side
+// q & 1.  The parity, not left/right, so that the node column shared by two
+// neighbouring grid cells stays in its accumulator lanes: walking on, a
+// finished grid cell's left node column is complete for these rows; its lanes
+// are written to LDS and cleared, and become the next right node column.
+//   At the end the workgroup adds, per window node and value, the at most four
+// fine rows (two where a pair of fine rows was added in registers) and two
+// column segments that touch it, in a fixed order.
 // No atomics: every sum has exactly one owner and a fixed order, so results
 // are identical run to run.  Tile windows overlap by two node rows/columns;
 // k_combine adds the at most 2 x 2 window partials of each node in a fixed
 // tile order.  Sums accumulate with fused multiply-add, which changes the
 // rounding of the sequential sums only.
+#include <cmath>
+#include <type_traits>
+
 #include "ereb_internal.h"
 
 namespace ereb {
 
-constexpr int CH = 256;      // markers per LDS chunk
-constexpr int CHP = CH + 1;  // padded stride: fields of one marker in different banks
-constexpr int NCF = 2 * FINE;  // fine cells in one basic column of a tile
-constexpr int NLF = 18;        // property values staged per marker
-// Partials of one column: value q of grid G for (half column h, corner row
-// ci, corner column cj, fine row fi) at
-//   part[poff + q*PQ + h*PH + ci*PCI + cj*PCJ + fi].
-// In the combine, the 16 lanes that read one value hold 8 fine rows 2 apart
-// and the two corner columns: fine rows 2 doubles apart and an odd corner
-// column stride (13 doubles) put the 16 reads in 32 distinct LDS banks.
-constexpr int PCJ = FINE + 1, PCI = 2 * PCJ, PH = 2 * PCI, PQ = 2 * PH;
-constexpr int NPART = NSUM * PQ;
+constexpr int NSEG = 2;              // column segments of a tile, a wavefront each per 4 fine rows
+constexpr int SEGC = FINE / NSEG;    // fine columns of a segment (even)
+constexpr int NRB = FINE / 4;        // wavefronts on top of each other (4 fine rows each)
+constexpr int SCAT_NW = NSEG * NRB;  // wavefronts of a workgroup
+// wavefronts a SIMD whose registers fit (no spills: a spilled value's reload
+// waits for every load in flight)
+constexpr int scat_waves(bool mixed, bool typed) {
+    return typed && mixed ? 5 : 4;
+}
+static_assert(SEGC % 2 == 0 && FINE % 4 == 0, "segment shape");
 
-// staged property indices
-enum {
-    L_ETATOTAL = 0, L_ETAVP, L_INVGGG, L_SXY, L_COHES, L_TENS, L_FRICT,  // basic
-    L_RHOTOTAL, L_RHOF, L_KTOTAL, L_PHIM, L_ETAFKPHI,                    // Vx, Vy
-    L_SXX, L_RHOCP, L_ALPHAS, L_ALPHAF, L_HR, L_TKRHOCP                  // P
+// Quads of property values (B operands):
+//   N1 etatotal etavp sxy -(1)   N2 rhototal ktotal etafkphi phi
+//   N3 sxx tkrhocp rhocptotal hrtotal
+// typed markers (ScatterArgs::typed): I, the indicators of the three types;
+// the seven type-derived values' sums and the weight sum are combinations of
+// the three indicators' sums.  Otherwise
+//   T1 tens frict 1/G cohes      T2 rhof alphas alphaf 1
+// Accumulator a (one double a lane) sums quad QUAD[a] on grid GRID[a]; column
+// j is slot SLOT[a] >> 4 j & 15 of that grid's sums in LDS (15: none).  The
+// slots are the SUM order without the typed values, then the three
+// indicators; for untyped markers the SUM order.
+enum { N1 = 0, N2, N3, T1, T2, I = T1 };
+template <bool TYPED> struct Plan;
+template <> struct Plan<true> {
+    static constexpr int nquad = 4, nacc = 9;
+    static constexpr int nsum[4] = {6, 7, 7, 9};
+    static constexpr int GRID[nacc] = {0, 0, 1, 1, 2, 2, 3, 3, 3};
+    static constexpr int QUAD[nacc] = {N1, I, N2, I, N2, I, N2, N3, I};
+    // basic eta etavp sxy | Vx, Vy rho k etafk phi | P rho phi sxx tk rhocp hr
+    static constexpr uint32_t SLOT[nacc] = {0xf210, 0xf543, 0x3210, 0xf654, 0x3210,
+                                            0xf654, 0x1ff0, 0x5432, 0xf876};
+};
+template <> struct Plan<false> {
+    static constexpr int nquad = 5, nacc = 10;
+    static constexpr int nsum[4] = {8, 6, 6, 10};
+    static constexpr int GRID[nacc] = {0, 0, 1, 1, 2, 2, 3, 3, 3, 3};
+    static constexpr int QUAD[nacc] = {N1, T1, N2, T2, N2, T2, N2, N3, T1, T2};
+    static constexpr uint32_t SLOT[nacc] = {0x7310, 0x4265, 0x3420, 0x5ff1, 0x3420,
+                                            0x5ff1, 0x8ff0, 0x4176, 0xf5ff, 0x932f};
 };
 
-// R is the type of the property vectors, the LDS staging and the per-fine-cell
-// sums: double in the Float64 form, float in the mixed form.  The marker
-// state (coordinates, temperature, porosity, stresses) is double in both.
+// Per-row sums in LDS, slot v of grid G for row c (a basic row on the grids
+// with basic y, whose two fine rows are added in registers; a fine row on the
+// others), side, node column slot: off + v*SV + side*SS + c*SC + slot.  Column
+// slots of segment s: SC / NSEG from s * SC / NSEG, the first for node column
+// s * SEGC / 2.  The strides spread a write (4 values, 4 rows, 2 sides) and a
+// read (8 columns, 4 rows) over the LDS banks.
+constexpr bool grid_prow(int G) { return G & 1; }   // staggered rows: Vx, P
+constexpr bool grid_pcol(int G) { return G >> 1; }  // staggered columns: Vy, P
+constexpr int SUM0[4] = {0, 8, 14, 20};             // first SUM of each grid
+constexpr int seg_cols(bool pcol) { return SEGC / 2 + (pcol ? 2 : 1); }
+template <bool TYPED, int G> struct PartShape {
+    static constexpr int cols = seg_cols(grid_pcol(G));
+    static constexpr int SC = NSEG * cols;
+    static constexpr int NR = grid_prow(G) ? FINE : TILE;
+    static constexpr int SS = NR * SC + 4, SV = 2 * SS + 1;
+    static constexpr int size = SV * Plan<TYPED>::nsum[G];
+    static constexpr int off() {
+        if constexpr (G == 0) return 0;
+        else return PartShape<TYPED, G - 1>::off() + PartShape<TYPED, G - 1>::size;
+    }
+};
+
 // Per-type values of the seven material vectors (E:659-665): 1/G (inv),
 // cohesion, tension, friction, fluid density, solid and fluid expansivity
 struct TypedTab {
@@ -91,12 +152,26 @@ __host__ static TypedTab typed_tab(const ereb_materials& M) {
     return T;
 }
 
+// every value finite in the vectors' precision: a combination of the types'
+// weight sums then equals the sum over the markers also where a type's weight
+// is zero
+template <class R>
+static bool tab_finite(const TypedTab& T) {
+    for (const auto& row : T.v)
+        for (double v : row)
+            if (!std::isfinite((R)v)) return false;
+    return true;
+}
+
 // row q of the table at type index t (0..2), by selects (no dynamic
 // indexing of the kernel argument)
 __device__ __forceinline__ double typed_at(const TypedTab& T, int q, int t) {
     return t == 0 ? T.v[q][0] : (t == 1 ? T.v[q][1] : T.v[q][2]);
 }
 
+// R is the type of the property vectors: double in the Float64 form, float in
+// the mixed form.  The marker state (coordinates, temperature, porosity,
+// stresses), the weights and the sums are double in both.
 template <class R>
 struct ScatterArgs {
     GeomK g;
@@ -110,421 +185,441 @@ struct ScatterArgs {
     // typed: 1/G, cohesion, tension, friction, fluid density and the two
     // expansivities are the material table values of the marker's type, as
     // the reference sets them (E:659-665, checked on the device by
-    // typed_refresh): read through tm from `tab` instead of seven vectors
+    // typed_refresh), all of them finite: tm is read instead of the seven
+    // vectors, whose sums follow from the types' weight sums and `tab`
     int typed;
     const int32_t* tm;
     TypedTab tab;
 };
 
-__device__ __forceinline__ double fma_r(double a, double b, double c) { return fma(a, b, c); }
-__device__ __forceinline__ float fma_r(float a, float b, float c) { return fmaf(a, b, c); }
-
-// per-node accumulators of the combine: plain double sums in the Float64 form,
-// compensated float sums (value + error term) in the mixed form
-template <class R> struct NodeAcc;
-template <> struct NodeAcc<double> {
-    double s[10];
-    __device__ void zero() {
-#pragma unroll
-        for (int q = 0; q < 10; ++q) s[q] = 0.0;
-    }
-    __device__ void add(int q, double v) { s[q] += v; }
-    __device__ double get(int q) const { return s[q]; }
-};
-template <> struct NodeAcc<float> {
-    float s[10], c[10];
-    __device__ void zero() {
-#pragma unroll
-        for (int q = 0; q < 10; ++q) s[q] = c[q] = 0.0f;
-    }
-    __device__ void add(int q, float v) { two_sum_add(s[q], c[q], v); }
-    __device__ double get(int q) const { return (double)s[q] + (double)c[q]; }
-};
-
-// per-grid SUM slot offset, partial offset and staged-property list (SUM
-// order of reset_interpolated_properties!, E:968-999).
-template <int G> struct GridSpec;
-template <> struct GridSpec<0> {  // basic: ETA0 ETA GGG SXY COH TEN FRI (+WT)
-    static constexpr int slot0 = 0, poff = 0, nf = 7;
-    static constexpr bool prow = false, pcol = false;
-    __device__ static constexpr int f(int q) {
-        return q == 0 ? L_ETATOTAL : q == 1 ? L_ETAVP : q == 2 ? L_INVGGG : q == 3 ? L_SXY
-             : q == 4 ? L_COHES : q == 5 ? L_TENS : L_FRICT;
-    }
-};
-template <> struct GridSpec<1> {  // Vx: RHOX RHOFX KX PHIX RX (+WTX)
-    static constexpr int slot0 = 8, poff = PQ * 8, nf = 5;
-    static constexpr bool prow = true, pcol = false;
-    __device__ static constexpr int f(int q) { return L_RHOTOTAL + q; }
-};
-template <> struct GridSpec<2> {  // Vy: RHOY RHOFY KY PHIY RY (+WTY)
-    static constexpr int slot0 = 14, poff = PQ * 14, nf = 5;
-    static constexpr bool prow = false, pcol = true;
-    __device__ static constexpr int f(int q) { return L_RHOTOTAL + q; }
-};
-template <> struct GridSpec<3> {  // P: RHO RHOCP ALPHA ALPHAF HR GGGP SXX TK PHI (+WTP)
-    static constexpr int slot0 = 20, poff = PQ * 20, nf = 9;
-    static constexpr bool prow = true, pcol = true;
-    __device__ static constexpr int f(int q) {
-        return q == 0 ? L_RHOTOTAL : q == 1 ? L_RHOCP : q == 2 ? L_ALPHAS : q == 3 ? L_ALPHAF
-             : q == 4 ? L_HR : q == 5 ? L_INVGGG : q == 6 ? L_SXX : q == 7 ? L_TKRHOCP
-             : L_PHIM;
-    }
-};
-
-template <class R>
-struct ScatterLDS {
-    R sf[NLF][CHP];
-    R sfr[4][CHP];  // dxmj/dx basic, dymi/dy basic, dxmj/dx P, dymi/dy P
-    R part[NPART];
-    double ax[4][WIN];   // tile window of the x, y, xp, yp axes
-    double typed[7][3];  // the typed material table (TypedTab)
+template <bool TYPED> struct ScatterLDS {
+    double part[PartShape<TYPED, 3>::off() + PartShape<TYPED, 3>::size];
+    double typed[7][3];  // the typed material table, in the vectors' precision
+    double ax[4][WIN];   // the window's x, xp, y and yp nodes
+    // where result lane l of accumulator a of row strip r goes in part, without
+    // the column slot; -1: nowhere
+    int32_t addr[NRB][Plan<TYPED>::nacc][64];
     int32_t fs[NFINE + 1];
 };
 
-// Values q = Q0 .. Q0+QN-1 of grid G's NQ = nf + 1 sums (q == nf is the weight
-// sum) for the task (fine cell fl of the column, corner column cj): lanes
-// 0..47 of one wavefront.  The marker values of iteration s + 1 are read from
-// LDS while iteration s accumulates.
-template <class R, int G, int Q0, int QN>
-__device__ __forceinline__ void tasks(ScatterLDS<R>& L, int lane, int f0, int c0, int cend) {
-    using S = GridSpec<G>;
-    constexpr int NQ = S::nf + 1;
-    static_assert(Q0 + QN <= NQ, "value range");
-    constexpr bool HASW = Q0 + QN == NQ;   // this part holds the weight sum
-    constexpr int NV = HASW ? QN - 1 : QN;  // staged property values read per marker
-    if (lane >= 2 * NCF) return;
-    const int fl = lane >> 1, cj = lane & 1;
-    const int k0 = max(L.fs[f0 + fl], c0) - c0, k1 = min(L.fs[f0 + fl + 1], cend) - c0;
-    const R* fa = S::pcol ? L.sfr[2] : L.sfr[0];
-    const R* fb = S::prow ? L.sfr[3] : L.sfr[1];
-    R s0[QN], s1[QN];  // corners (0, cj) and (1, cj)
+// lane G of the quad, in every lane of it
+template <int G>
+__device__ __forceinline__ int quad_bcast(int x) {
+    return __builtin_amdgcn_update_dpp(0, x, G * 0x55, 0xf, 0xf, true);
+}
+template <int G>
+__device__ __forceinline__ double quad_bcast(double x) {
+    const uint64_t u = (uint64_t)__double_as_longlong(x);
+    const uint32_t lo = (uint32_t)quad_bcast<G>((int)(uint32_t)u);
+    const uint32_t hi = (uint32_t)quad_bcast<G>((int)(uint32_t)(u >> 32));
+    return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+
+// a / d for d > 0 with r = 1 / d rounded once: the quotient rounded as by the
+// division (Markstein's final step: the residual of a * r by fma, times r; no
+// difference in 3e8 quotients of ten spacings), special cases by the divide's
+// fix-up instruction.  Four instructions instead of eleven.
+__device__ __forceinline__ double div_by(double a, double d, double r) {
+    const double q = a * r;
+    return __builtin_amdgcn_div_fixup(fma(fma(-q, d, a), r, q), d, a);
+}
+
+constexpr int QP_XOR1 = 0xB1, QP_XOR2 = 0x4E;  // quad_perm [1,0,3,2], [2,3,0,1]
+template <int CTRL>
+__device__ __forceinline__ double quad_swap(double x) {
+    const uint64_t u = (uint64_t)__double_as_longlong(x);
+    const uint32_t lo =
+        (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, CTRL, 0xf, 0xf, true);
+    const uint32_t hi =
+        (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), CTRL, 0xf, 0xf, true);
+    return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+
+// r[f] at lane t of a quad -> r[g] at lane j: the old r[j] of lane g
+__device__ __forceinline__ void quad_transpose(double (&r)[4], bool odd, bool high) {
 #pragma unroll
-    for (int q = 0; q < QN; ++q) s0[q] = s1[q] = R(0);
-    if (k0 < k1) {
-        R v[NV], a = fa[k0], b = fb[k0];
-#pragma unroll
-        for (int q = 0; q < NV; ++q) v[q] = L.sf[S::f(Q0 + q)][k0];
-        // two markers per trip in the mixed form (measured 4 µs faster there;
-        // in the Float64 form two gained nothing and four were 60% slower)
-        constexpr int UNROLL = sizeof(R) == 4 ? 2 : 1;
-#pragma unroll UNROLL
-        for (int s = k0; s < k1; ++s) {
-            const int sn = min(s + 1, k1 - 1);
-            R vn[NV];
-#pragma unroll
-            for (int q = 0; q < NV; ++q) vn[q] = L.sf[S::f(Q0 + q)][sn];
-            const R an = fa[sn], bn = fb[sn];
-            // weights order (i,j),(i+1,j),(i,j+1),(i+1,j+1) = (1-b)(1-a), b(1-a), (1-b)a, ba
-            const R wa = cj ? a : R(1) - a;
-            const R w0 = (R(1) - b) * wa, w1 = b * wa;
-#pragma unroll
-            for (int q = 0; q < NV; ++q) {
-                s0[q] = fma_r(v[q], w0, s0[q]);
-                s1[q] = fma_r(v[q], w1, s1[q]);
-            }
-            if (HASW) {
-                s0[QN - 1] += w0;
-                s1[QN - 1] += w1;
-            }
-#pragma unroll
-            for (int q = 0; q < NV; ++q) v[q] = vn[q];
-            a = an;
-            b = bn;
-        }
+    for (int f = 0; f < 4; f += 2) {
+        const double a = r[f], b = r[f + 1];
+        const double ax = quad_swap<QP_XOR1>(a), bx = quad_swap<QP_XOR1>(b);
+        r[f] = odd ? bx : a;
+        r[f + 1] = odd ? b : ax;
     }
-    const int h = fl >= FINE ? 1 : 0, fi = fl - h * FINE;
-    R* p = &L.part[S::poff + Q0 * PQ + h * PH + cj * PCJ + fi];
 #pragma unroll
-    for (int q = 0; q < QN; ++q) {
-        p[q * PQ] = s0[q];
-        p[q * PQ + PCI] = s1[q];
+    for (int f = 0; f < 2; ++f) {
+        const double a = r[f], b = r[f + 2];
+        const double ax = quad_swap<QP_XOR2>(a), bx = quad_swap<QP_XOR2>(b);
+        r[f] = high ? bx : a;
+        r[f + 2] = high ? b : ax;
     }
 }
 
-// node (r, c) of grid G adds values Q0 .. Q0+QN-1 of the partials of the fine
-// cells of basic column k that touch it: fine columns 2k + h, fine rows
-// fi_lo .. fi_lo + 3
-template <class R, int G, int Q0, int QN>
-__device__ __forceinline__ void combine(const ScatterLDS<R>& L, NodeAcc<R>& acc, int r, int c,
-                                        int k) {
-    using S = GridSpec<G>;
-    const int fi_lo = S::prow ? 2 * r - 3 : 2 * r - 2;
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        const int fj = 2 * k + h;
-        const int cj = c - (S::pcol ? (fj + 1) >> 1 : fj >> 1);
-        if (cj < 0 || cj > 1) continue;
-        R v[4][QN];
-#pragma unroll
-        for (int d = 0; d < 4; ++d) {
-            const int fi = min(max(fi_lo + d, 0), FINE - 1);  // clamped; skipped below
-            const int ci = 1 - (d >> 1);  // = r - (grid row of fine row fi)
-            const R* p = &L.part[S::poff + Q0 * PQ + h * PH + ci * PCI + cj * PCJ + fi];
-#pragma unroll
-            for (int q = 0; q < QN; ++q) v[d][q] = p[q * PQ];
-        }
-#pragma unroll
-        for (int d = 0; d < 4; ++d) {
-            const int fi = fi_lo + d;
-            if (fi < 0 || fi >= FINE) continue;
-#pragma unroll
-            for (int q = 0; q < QN; ++q) acc.add(q, v[d][q]);
-        }
-    }
-}
-
-template <class R, int G, int Q0, int QN>
-__device__ __forceinline__ void write_part(double* part, int tile, const NodeAcc<R>& acc,
-                                           int lane) {
-    using S = GridSpec<G>;
-    double* p = part + ((size_t)tile * NSUM + S::slot0 + Q0) * 64 + lane;
-#pragma unroll
-    for (int q = 0; q < QN; ++q) p[(size_t)q * 64] = acc.get(q);
-}
-
-// Inputs of one marker, loaded one chunk ahead of their use so that the
-// global-memory latency of the gather through perm overlaps the previous
-// chunk's task and combine phases.  The two halves of the workgroup load
-// half of each marker's inputs each (part 0: xm, ym, phim, sxxm, sxym,
-// etavp, 1/G, cohesion, tension, friction; part 1: rhofluid, alphasolid,
-// alphafluid and the 7 marker properties, which the sort's key pass
-// evaluated in storage order).  Values are held as double (float inputs of
-// the mixed form convert exactly).
-constexpr int NRAW = 10;
-
-template <class R>
-__device__ __forceinline__ void load_raw(const ScatterArgs<R>& A, const ScatterLDS<R>& L,
-                                         int part, uint32_t m, double (&v)[NRAW]) {
-    if (part == 0) {
-        v[0] = A.xm[m];
-        v[1] = A.ym[m];
-        v[2] = A.phim[m];
-        v[3] = A.sxx[m];
-        v[4] = A.sxy[m];
-        v[5] = A.etavp[m];
-        if (A.typed) {
-            const int t = min(max(A.tm[m], 1), 3) - 1;
-            v[6] = L.typed[0][t];
-            v[7] = L.typed[1][t];
-            v[8] = L.typed[2][t];
-            v[9] = L.typed[3][t];
-        } else {
-            v[6] = A.invggg[m];
-            v[7] = A.cohes[m];
-            v[8] = A.tens[m];
-            v[9] = A.frict[m];
-        }
-    } else {
-        if (A.typed) {
-            const int t = min(max(A.tm[m], 1), 3) - 1;
-            v[0] = L.typed[4][t];
-            v[1] = L.typed[5][t];
-            v[2] = L.typed[6][t];
-        } else {
-            v[0] = A.rhof[m];
-            v[1] = A.alphas[m];
-            v[2] = A.alphaf[m];
-        }
-        v[3] = A.rhototal[m];
-        v[4] = A.rhocptotal[m];
-        v[5] = A.etatotal[m];
-        v[6] = A.hrtotal[m];
-        v[7] = A.ktotal[m];
-        v[8] = A.tkrhocp[m];
-        v[9] = A.etafkphi[m];
-    }
-}
-
-// one half of a marker's staged values into LDS slot t: part 0 also the
-// stencil fractions.  (j0, i0): 0-based first basic column and row of the
-// tile.  Every marker of the tile has jb - 1, ib - 1 in [0, TILE) and
-// jp - 1, ip - 1 in [0, TILE] relative to them (its fine key was derived
-// from these cells).
-template <class R>
-__device__ __forceinline__ void stage_raw(const ScatterArgs<R>& A, ScatterLDS<R>& L, int part,
-                                          int t, const double (&v)[NRAW], int j0, int i0) {
-    if (part == 0) {
-        const double x = v[0], y = v[1];
-        const Cells cl = marker_cells(A.g, x, y);
-        // fractions in double from the double coordinates, then rounded to R
-        L.sfr[0][t] = (R)((x - L.ax[0][cl.jb - 1 - j0]) / A.g.dx);
-        L.sfr[1][t] = (R)((y - L.ax[1][cl.ib - 1 - i0]) / A.g.dy);
-        L.sfr[2][t] = (R)((x - L.ax[2][cl.jp - 1 - j0]) / A.g.dx);
-        L.sfr[3][t] = (R)((y - L.ax[3][cl.ip - 1 - i0]) / A.g.dy);
-        L.sf[L_PHIM][t] = (R)v[2];
-        L.sf[L_SXX][t] = (R)v[3];
-        L.sf[L_SXY][t] = (R)v[4];
-        L.sf[L_ETAVP][t] = (R)v[5];
-        L.sf[L_INVGGG][t] = (R)v[6];
-        L.sf[L_COHES][t] = (R)v[7];
-        L.sf[L_TENS][t] = (R)v[8];
-        L.sf[L_FRICT][t] = (R)v[9];
-    } else {
-        L.sf[L_RHOF][t] = (R)v[0];
-        L.sf[L_ALPHAS][t] = (R)v[1];
-        L.sf[L_ALPHAF][t] = (R)v[2];
-        L.sf[L_RHOTOTAL][t] = (R)v[3];
-        L.sf[L_RHOCP][t] = (R)v[4];
-        L.sf[L_ETATOTAL][t] = (R)v[5];
-        L.sf[L_HR][t] = (R)v[6];
-        L.sf[L_KTOTAL][t] = (R)v[7];
-        L.sf[L_TKRHOCP][t] = (R)v[8];
-        L.sf[L_ETAFKPHI][t] = (R)v[9];
-    }
-}
-
-// Chunks of a tile: basic column k, markers [c0, cend) with cend - c0 <= CH.
-// k == TILE marks the end.  All fields are wave-uniform.
-struct Chunk {
-    int k, c0, cend;
+// A chunk's loaded values: the lane's marker's, by quad
+template <class R, bool TYPED> struct ChunkData {
+    double sxy, sxx, phi, x, y;
+    R etatotal, etavp, rhototal, ktotal, etafkphi, tkrhocp, rhocptotal, hrtotal;
+    R tens, frict, invggg, cohes, rhof, alphas, alphaf;  // untyped
+    int32_t tm;                                          // typed
+    int32_t fj;                                          // fine column, -1: no marker
 };
 
-template <class R>
-__device__ __forceinline__ Chunk chunk_from(const ScatterLDS<R>& L, int k, int c0) {
-    for (; k < TILE; ++k) {
-        const int ce = __builtin_amdgcn_readfirstlane(L.fs[(k + 1) * NCF]);
-        if (c0 < ce) return Chunk{k, c0, min(c0 + CH, ce)};
-        if (k + 1 < TILE) c0 = max(c0, __builtin_amdgcn_readfirstlane(L.fs[(k + 1) * NCF]));
+// loads of the lane's marker m
+template <class R, bool TYPED>
+__device__ __forceinline__ void load_marker(const ScatterArgs<R>& A, uint32_t mk, int fj,
+                                            ChunkData<R, TYPED>& D) {
+    D = ChunkData<R, TYPED>{};
+    D.fj = fj;
+    if (fj < 0) return;
+    const size_t m = mk;
+    D.x = A.xm[m];
+    D.y = A.ym[m];
+    if constexpr (TYPED) D.tm = A.tm[m];
+    D.etatotal = A.etatotal[m];
+    D.etavp = A.etavp[m];
+    D.sxy = A.sxy[m];
+    D.rhototal = A.rhototal[m];
+    D.ktotal = A.ktotal[m];
+    D.etafkphi = A.etafkphi[m];
+    D.phi = A.phim[m];
+    D.sxx = A.sxx[m];
+    D.tkrhocp = A.tkrhocp[m];
+    D.rhocptotal = A.rhocptotal[m];
+    D.hrtotal = A.hrtotal[m];
+    if constexpr (!TYPED) {
+        D.tens = A.tens[m];
+        D.frict = A.frict[m];
+        D.invggg = A.invggg[m];
+        D.cohes = A.cohes[m];
+        D.rhof = A.rhof[m];
+        D.alphas = A.alphas[m];
+        D.alphaf = A.alphaf[m];
     }
-    return Chunk{TILE, 0, 0};
 }
 
-template <class R>
-__device__ __forceinline__ Chunk chunk_next(const ScatterLDS<R>& L, const Chunk& c) {
-    return c.k < TILE ? chunk_from(L, c.k, c.cend) : c;
+// addresses of strip rb's results (ScatterLDS::addr)
+template <bool TYPED, int A0 = 0>
+__device__ __forceinline__ void result_addr(ScatterLDS<TYPED>& L, int lane, int rb) {
+    using P = Plan<TYPED>;
+    if constexpr (A0 < P::nacc) {
+        using PS = PartShape<TYPED, P::GRID[A0]>;
+        constexpr bool prow = grid_prow(P::GRID[A0]);
+        const int j = lane & 3, b = lane >> 2 & 3, side = lane >> 4 & 1;
+        const int s = (int)(P::SLOT[A0] >> (4 * j)) & 15;
+        const int c = prow ? 4 * rb + b : 2 * rb + (b >> 1);
+        const bool used = s != 15 && (prow || !(b & 1));
+        L.addr[rb][A0][lane] =
+            used ? PS::off() + s * PS::SV + side * PS::SS + c * PS::SC : -1;
+        result_addr<TYPED, A0 + 1>(L, lane, rb);
+    }
 }
 
-template <class R>
-__device__ __forceinline__ uint32_t chunk_perm(const ScatterArgs<R>& A, const Chunk& c, int t) {
-    return (c.k < TILE && t < c.cend - c.c0) ? A.perm[c.c0 + t] : 0u;
+// node column slot `slot` of the accumulators of the grids with column kind
+// PCOL: the lanes of its parity (mine) write their sums and start over.  All
+// LDS reads first, so that one wait covers them.
+template <bool TYPED, bool PCOL>
+__device__ __forceinline__ void write_col(ScatterLDS<TYPED>& L, double (&acc)[Plan<TYPED>::nacc],
+                                          int lane, int rb, int slot, bool mine) {
+    using P = Plan<TYPED>;
+    int at[P::nacc];
+    int2 other[P::nacc];
+#pragma unroll
+    for (int a = 0; a < P::nacc; ++a) {
+        if (grid_pcol(P::GRID[a]) != PCOL) continue;
+        at[a] = L.addr[rb][a][lane];
+        if (grid_prow(P::GRID[a])) continue;
+        // the basic row's other fine row (lane ^ 4)
+        const uint64_t u = (uint64_t)__double_as_longlong(acc[a]);
+        other[a].x = __builtin_amdgcn_ds_swizzle((int)(uint32_t)u, 0x101F);
+        other[a].y = __builtin_amdgcn_ds_swizzle((int)(uint32_t)(u >> 32), 0x101F);
+    }
+#pragma unroll
+    for (int a = 0; a < P::nacc; ++a) {
+        if (grid_pcol(P::GRID[a]) != PCOL) continue;
+        double v = acc[a];
+        if (!grid_prow(P::GRID[a]))
+            v += __longlong_as_double(
+                (long long)(((uint64_t)(uint32_t)other[a].y << 32) | (uint32_t)other[a].x));
+        if (mine && at[a] >= 0) L.part[at[a] + slot] = v;
+        acc[a] = mine ? 0.0 : acc[a];
+    }
 }
 
-// Wavefronts per workgroup: 8 in the Float64 form (two per grid, each thread
-// loading half of a marker's inputs; 116 VGPRs, 4 waves per SIMD), 4 in the
-// mixed form (one per grid, each thread loading a whole marker; its smaller
-// LDS footprint already fits 4 workgroups per CU, and halving the work per
-// thread there measured 36% slower).
-template <class R> struct ScatterShape;
-template <> struct ScatterShape<double> { static constexpr int NW = 8; };
-template <> struct ScatterShape<float> { static constexpr int NW = 4; };
+// Where the sums of window node (r, c) of grid G lie in part: the rows above
+// (their side 1) and below (side 0) the node, the segments that hold its
+// column, in this order; out-of-range terms point at a term in range, unused
+template <bool TYPED, int G> struct NodeTerms {
+    using PS = PartShape<TYPED, G>;
+    static constexpr int n = grid_prow(G) ? 2 : 1;  // rows a side
+    static constexpr int N = 2 * n * NSEG;
+    int at[N];
+    bool ok[N];
+    __device__ __forceinline__ NodeTerms(int r, int c) {
+        const int r1 = grid_prow(G) ? 2 * r - 3 : r - 1;
+#pragma unroll
+        for (int d = 0; d < 2 * n; ++d) {
+            const int row = r1 + d, side = d < n ? 1 : 0;
+#pragma unroll
+            for (int g = 0; g < NSEG; ++g) {
+                const int slot = c - g * (SEGC / 2), i = d * NSEG + g;
+                ok[i] = row >= 0 && row < PS::NR && slot >= 0 && slot < PS::cols;
+                at[i] = PS::off() + (ok[i] ? side * PS::SS + row * PS::SC + g * PS::cols + slot : 0);
+            }
+        }
+    }
+    __device__ __forceinline__ double sum(const ScatterLDS<TYPED>& L, int v) const {
+        double t[N], s = 0.0;
+#pragma unroll
+        for (int i = 0; i < N; ++i) t[i] = L.part[at[i] + v * PS::SV];
+#pragma unroll
+        for (int i = 0; i < N; ++i) s += ok[i] ? t[i] : 0.0;
+        return s;
+    }
+};
 
-template <class R>
-__global__ __launch_bounds__(ScatterShape<R>::NW * 64, 2) void k_scatter(ScatterArgs<R> A) {
-    constexpr int NW = ScatterShape<R>::NW, NTHR = NW * 64;
-    constexpr int NSET = NW == 8 ? 1 : 2;  // input halves per thread
-    __shared__ ScatterLDS<R> L;
+// one node's sums of one grid: value v (the grid's own numbering) of `out`
+// from slot s; from the three indicators' sums w
+template <bool TYPED, int G> struct NodeOut {
+    const ScatterLDS<TYPED>& L;
+    const NodeTerms<TYPED, G> T;
+    double* out;
+    __device__ __forceinline__ NodeOut(const ScatterLDS<TYPED>& L_, double* o, int r, int c)
+        : L(L_), T(r, c), out(o + (size_t)SUM0[G] * 64) {}
+    __device__ __forceinline__ void put(int v, int s) const { out[v * 64] = T.sum(L, s); }
+    // the weight sum (value v) and the typed values of table rows q: the
+    // indicators' sums are in slots s..s+2
+    double w[3];
+    __device__ __forceinline__ void types(int v, int s) {
+#pragma unroll
+        for (int e = 0; e < 3; ++e) w[e] = T.sum(L, s + e);
+        out[v * 64] = (w[0] + w[1]) + w[2];
+    }
+    __device__ __forceinline__ void typed(int v, int q) const {
+        out[v * 64] = fma(L.typed[q][2], w[2], fma(L.typed[q][1], w[1], L.typed[q][0] * w[0]));
+    }
+};
+
+// the window's 30 sums, split over the workgroup's wavefronts by the LDS terms
+// they add
+template <bool TYPED>
+__device__ __forceinline__ void window_sums(const ScatterLDS<TYPED>& L, double* out, int wave,
+                                            int lane) {
+    static_assert(SCAT_NW == 6, "the split below");
+    // the lane's node: neighbouring lanes read neighbouring column slots
+    const int c = lane & 7, r = lane >> 3;
+    out += 8 * c + r;
+    if constexpr (TYPED) {
+        // typed table rows: 1/G, cohesion, tension, friction, rhof, alphas, alphaf
+        if (wave == 0) {  // basic ETA0 ETA (GGG) SXY (COH TEN FRI) WT
+            NodeOut<true, 0> o(L, out, r, c);
+            o.put(0, 0);
+            o.put(1, 1);
+            o.put(3, 2);
+            o.types(7, 3);
+            o.typed(2, 0);
+            o.typed(4, 1);
+            o.typed(5, 2);
+            o.typed(6, 3);
+        } else if (wave == 1) {  // Vx RHOX (RHOFX) KX PHIX RX WTX
+            NodeOut<true, 1> o(L, out, r, c);
+            o.put(0, 0);
+            o.put(2, 1);
+            o.put(3, 3);
+            o.put(4, 2);
+        } else if (wave == 2) {
+            NodeOut<true, 1> o(L, out, r, c);
+            o.types(5, 4);
+            o.typed(1, 4);
+        } else if (wave == 3) {  // Vy
+            NodeOut<true, 2> o(L, out, r, c);
+            o.put(0, 0);
+            o.put(2, 1);
+            o.put(3, 3);
+            o.put(4, 2);
+            o.types(5, 4);
+            o.typed(1, 4);
+        } else if (wave == 4) {  // P RHO RHOCP (ALPHA ALPHAF) HR (GGGP) SXX TK PHI WTP
+            NodeOut<true, 3> o(L, out, r, c);
+            o.put(0, 0);
+            o.put(8, 1);
+            o.put(6, 2);
+            o.put(7, 3);
+        } else {
+            NodeOut<true, 3> o(L, out, r, c);
+            o.put(1, 4);
+            o.put(4, 5);
+            o.types(9, 6);
+            o.typed(2, 5);
+            o.typed(3, 6);
+            o.typed(5, 0);
+        }
+    } else {
+        auto all = [&](auto o, int v0, int v1) {
+            for (int v = v0; v < v1; ++v) o.put(v, v);
+        };
+        if (wave == 0) all(NodeOut<false, 0>(L, out, r, c), 0, 8);
+        else if (wave == 1) all(NodeOut<false, 1>(L, out, r, c), 0, 3);
+        else if (wave == 2) all(NodeOut<false, 1>(L, out, r, c), 3, 6);
+        else if (wave == 3) all(NodeOut<false, 2>(L, out, r, c), 0, 6);
+        else if (wave == 4) all(NodeOut<false, 3>(L, out, r, c), 0, 5);
+        else all(NodeOut<false, 3>(L, out, r, c), 5, 10);
+    }
+}
+
+template <class R, bool TYPED>
+__global__ __launch_bounds__(SCAT_NW * 64, scat_waves(sizeof(R) == 4, TYPED)) void k_scatter(ScatterArgs<R> A) {
+    using P = Plan<TYPED>;
+    __shared__ ScatterLDS<TYPED> L;
     // XCD-contiguous: vertically neighbouring tiles (consecutive numbers)
     // read adjacent runs of the same marker columns
     const int tile = (int)xcd_block();
-    const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
-    const int part = NW == 8 ? wave >> 2 : 0, ts = t % CH;  // first input half, marker slot
-    const int r = lane & 7, c = lane >> 3;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int rb = wave % NRB, seg = wave / NRB;
+    const int t = lane & 3, b = lane >> 2 & 3, k = lane >> 4;
     const int j0 = (tile / A.nty) * TILE, i0 = (tile % A.nty) * TILE;
-    for (int i = t; i <= NFINE; i += NTHR) L.fs[i] = A.fstart[(size_t)tile * NFINE + i];
-    if (t < 21) L.typed[t / 3][t % 3] = A.tab.v[t / 3][t % 3];
-    if (t < 4 * WIN) {
-        const int a = t / WIN, k = t % WIN;
-        const double* axis = a == 0 ? A.g.x : a == 1 ? A.g.y : a == 2 ? A.g.xp : A.g.yp;
-        const int n = a == 0 ? A.g.Nx : a == 1 ? A.g.Ny : a == 2 ? A.g.Nx1 : A.g.Ny1;
-        const int k0 = (a & 1) ? i0 : j0;
-        L.ax[a][k] = k0 + k < n ? axis[k0 + k] : 0.0;
+    for (int i = tid; i <= NFINE; i += SCAT_NW * 64)
+        L.fs[i] = A.fstart[(size_t)tile * NFINE + i];
+    if (TYPED && tid < 21) L.typed[tid / 3][tid % 3] = (double)(R)A.tab.v[tid / 3][tid % 3];
+    if (tid < 4 * WIN) {
+        const int e = tid / WIN, w = tid % WIN;
+        const double* axis = e == 0 ? A.g.x : e == 1 ? A.g.xp : e == 2 ? A.g.y : A.g.yp;
+        const int n = e == 0 ? A.g.Nx : e == 1 ? A.g.Nx1 : e == 2 ? A.g.Ny : A.g.Ny1;
+        L.ax[e][w] = axis[min((e < 2 ? j0 : i0) + w, n - 1)];
     }
+    if (seg == 0) result_addr<TYPED>(L, lane, rb);
     __syncthreads();
-    NodeAcc<R> acc;
-    acc.zero();
 
-    Chunk cur = chunk_from(L, 0, __builtin_amdgcn_readfirstlane(L.fs[0]));
-    Chunk nx = chunk_next(L, cur);
-    double raw[NSET][NRAW];
-    // the first chunk is staged before the loop; each iteration then stages
-    // the next chunk while its combine runs (the combine reads the partials,
-    // the staging writes the staged values), two barriers per chunk
-    if (cur.k < TILE && ts < cur.cend - cur.c0) {
-        const uint32_t m = chunk_perm(A, cur, ts);
+    const int fi = 4 * rb + b;  // the block's fine row
+    const double dx = A.g.dx, dy = A.g.dy, rdx = A.g.idx, rdy = A.g.idy;
+    const bool ls = !(t & 1);  // the A row's node row: upper (weight 1 - f) or lower (f)
+    double acc[P::nacc];
 #pragma unroll
-        for (int q = 0; q < NSET; ++q) load_raw(A, L, part + q, m, raw[q]);
+    for (int a = 0; a < P::nacc; ++a) acc[a] = 0.0;
+
+    const int f0 = seg * SEGC, f1 = f0 + SEGC;
+    // groups of the segment's fine columns before its column q: pre[q]; all
+    // wave-uniform
+    int pre[SEGC + 1];
+    pre[0] = 0;
 #pragma unroll
-        for (int q = 0; q < NSET; ++q) stage_raw(A, L, part + q, ts, raw[q], j0, i0);
+    for (int q = 0; q < SEGC; ++q) {
+        const int n = L.fs[(f0 + q) * FINE + fi + 1] - L.fs[(f0 + q) * FINE + fi];
+        const int nmax =
+            max(max(__builtin_amdgcn_readlane(n, 0), __builtin_amdgcn_readlane(n, 4)),
+                max(__builtin_amdgcn_readlane(n, 8), __builtin_amdgcn_readlane(n, 12)));
+        pre[q + 1] = pre[q] + ((nmax + 3) >> 2);
     }
-    uint32_t pnx = chunk_perm(A, nx, ts);
+    // the lane's marker of the chunk at group s0: its fine column in fj (-1:
+    // none).  A chunk takes a run of each cell's markers, 4 a group; it is dealt
+    // so that the lanes of a quad (one a group) take neighbouring markers.
+    auto marker = [&](int s0, int& fj) {
+        const int s = s0 + t;
+        int q = 0, p = 0, pn = pre[1];
+#pragma unroll
+        for (int e = 1; e < SEGC; ++e) {
+            q = s >= pre[e] ? e : q;
+            p = s >= pre[e] ? pre[e] : p;
+            pn = s >= pre[e] ? pre[e + 1] : pn;
+        }
+        // the chunk's groups of this column: first g0 of it, ng of them
+        const int g0 = max(p, s0), ng = min(pn, s0 + 4) - g0;
+        const int a = L.fs[(f0 + q) * FINE + fi], o = 4 * (g0 - p) + k * ng + (s - g0);
+        const bool on = s < pre[SEGC] && o < L.fs[(f0 + q) * FINE + fi + 1] - a;
+        fj = on ? f0 + q : -1;
+        return on ? A.perm[a + o] : 0u;
+    };
+    // fine column `col` is done: the grid cells that end with it
+    int col = f0, end = pre[1];  // end: the group after col's last
+    auto next_col = [&]() {
+        const int pb = col >> 1, c = pb - seg * (SEGC / 2);
+        const bool mine = (lane >> 5) == (pb & 1);
+        if (col & 1)
+            write_col<TYPED, false>(L, acc, lane, rb, seg * seg_cols(false) + c, mine);
+        else
+            write_col<TYPED, true>(L, acc, lane, rb, seg * seg_cols(true) + c, mine);
+        ++col;
+        int e = 0;
+#pragma unroll
+        for (int q = 1; q <= SEGC; ++q) e = col - f0 == q - 1 ? pre[q] : e;
+        end = e;
+    };
+    while (col < f1 && end == 0) next_col();  // empty columns before the first marker
+    ChunkData<R, TYPED> D;
+    int fjx;
+    {
+        const uint32_t m = marker(0, fjx);
+        load_marker<R, TYPED>(A, m, fjx, D);
+    }
+    uint32_t mx = marker(4, fjx);
+    for (int s0 = 0; s0 < pre[SEGC]; s0 += 4) {
+        // this chunk's values out of the load registers, the next one's into
+        // them, then this chunk's products
+        const int cj = max(D.fj, 0);
+        const double xb = L.ax[0][cj >> 1], xp = L.ax[1][(cj + 1) >> 1];
+        // read here, not held in registers across the chunks
+        int ci = fi;
+        asm volatile("" : "+v"(ci));
+        const double yb = L.ax[2][ci >> 1], yp = L.ax[3][(ci + 1) >> 1];
+        double fxb = div_by(D.x - xb, dx, rdx), fxp = div_by(D.x - xp, dx, rdx);
+        double fyb = div_by(D.y - yb, dy, rdy), fyp = div_by(D.y - yp, dy, rdy);
+        int tm = D.fj >= 0 ? min(max(D.tm, 1), 3) : 0;
+        // done here, before the loads below (as the transposes)
+        asm volatile("" : "+v"(fxb), "+v"(fxp), "+v"(fyb), "+v"(fyp), "+v"(tm));
+        double q[P::nquad][4];
+        {
+            const double one = D.fj >= 0 ? 1.0 : 0.0;
+            const double raw[5][4] = {
+                {(double)D.etatotal, (double)D.etavp, D.sxy, TYPED ? 0.0 : one},
+                {(double)D.rhototal, (double)D.ktotal, (double)D.etafkphi, D.phi},
+                {D.sxx, (double)D.tkrhocp, (double)D.rhocptotal, (double)D.hrtotal},
+                {(double)D.tens, (double)D.frict, (double)D.invggg, (double)D.cohes},
+                {(double)D.rhof, (double)D.alphas, (double)D.alphaf, one}};
+#pragma unroll
+            for (int u = 0; u < (TYPED ? 3 : 5); ++u) {
+#pragma unroll
+                for (int f = 0; f < 4; ++f) q[u][f] = raw[u][f];
+                quad_transpose(q[u], t & 1, t & 2);
+                // done here: the selects would otherwise move into the groups
+                // below and hold twice the registers until then
+#pragma unroll
+                for (int f = 0; f < 4; ++f) asm volatile("" : "+v"(q[u][f]));
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        load_marker<R, TYPED>(A, mx, fjx, D);
+        mx = marker(s0 + 8, fjx);
+        __builtin_amdgcn_sched_barrier(0);
+        auto group = [&](auto gc) {
+            constexpr int g = decltype(gc)::value;
+            if (s0 + g >= pre[SEGC]) return;
+            // 1 - f or f: the A row's node column, of the left one's parity or
+            // not, and its node row, upper or lower
+            const double axb = quad_bcast<g>(fxb), axp = quad_bcast<g>(fxp);
+            const double ayb = quad_bcast<g>(fyb), ayp = quad_bcast<g>(fyp);
+            const bool lb = ((t >> 1 ^ col >> 1) & 1) == 0, lp = ((t >> 1 ^ (col + 1) >> 1) & 1) == 0;
+            const double wxb = lb ? 1.0 - axb : axb, wxp = lp ? 1.0 - axp : axp;
+            const double wyb = ls ? 1.0 - ayb : ayb, wyp = ls ? 1.0 - ayp : ayp;
+            const double w[4] = {wyb * wxb, wyp * wxb, wyb * wxp, wyp * wxp};
+            if constexpr (TYPED) q[I][g] = quad_bcast<g>(tm) == t + 1 ? 1.0 : 0.0;
+#pragma unroll
+            for (int e = 0; e < P::nacc; ++e)
+                acc[e] = __builtin_amdgcn_mfma_f64_4x4x4f64(w[P::GRID[e]], q[P::QUAD[e]][g],
+                                                            acc[e], 0, 0, 0);
+            while (col < f1 && s0 + g + 1 == end) next_col();
+        };
+        group(std::integral_constant<int, 0>{});
+        group(std::integral_constant<int, 1>{});
+        group(std::integral_constant<int, 2>{});
+        group(std::integral_constant<int, 3>{});
+    }
+    {   // the columns still open at the segment's end: the right column of the
+        // last basic column cell, both columns of the last P column cell
+        const bool even = (lane >> 5) == (f1 >> 1 & 1);  // parity of column f1 / 2
+        const int c = SEGC / 2;
+        write_col<TYPED, false>(L, acc, lane, rb, seg * seg_cols(false) + c, even);
+        write_col<TYPED, true>(L, acc, lane, rb, seg * seg_cols(true) + c + (even ? 0 : 1), true);
+    }
     __syncthreads();
-    while (cur.k < TILE) {
-        // ---- 1. loads of the next chunk's markers, perm of the one after ----
-        const Chunk nx2 = chunk_next(L, nx);
-        if (nx.k < TILE && ts < nx.cend - nx.c0) {
-#pragma unroll
-            for (int q = 0; q < NSET; ++q) load_raw(A, L, part + q, pnx, raw[q]);
-        }
-        pnx = chunk_perm(A, nx2, ts);
-        // ---- 2. (fine cell, corner column) partials: wavefronts g and g + 4
-        // own the first and second half of grid g's sums ---------------------
-        const int f0 = cur.k * NCF;
-        if constexpr (NW == 4) {
-            switch (wave) {
-                case 0: tasks<R, 0, 0, 8>(L, lane, f0, cur.c0, cur.cend); break;
-                case 1: tasks<R, 1, 0, 6>(L, lane, f0, cur.c0, cur.cend); break;
-                case 2: tasks<R, 2, 0, 6>(L, lane, f0, cur.c0, cur.cend); break;
-                default: tasks<R, 3, 0, 10>(L, lane, f0, cur.c0, cur.cend); break;
-            }
-        } else switch (wave) {
-            case 0: tasks<R, 0, 0, 4>(L, lane, f0, cur.c0, cur.cend); break;
-            case 1: tasks<R, 1, 0, 3>(L, lane, f0, cur.c0, cur.cend); break;
-            case 2: tasks<R, 2, 0, 3>(L, lane, f0, cur.c0, cur.cend); break;
-            case 3: tasks<R, 3, 0, 5>(L, lane, f0, cur.c0, cur.cend); break;
-            case 4: tasks<R, 0, 4, 4>(L, lane, f0, cur.c0, cur.cend); break;
-            case 5: tasks<R, 1, 3, 3>(L, lane, f0, cur.c0, cur.cend); break;
-            case 6: tasks<R, 2, 3, 3>(L, lane, f0, cur.c0, cur.cend); break;
-            default: tasks<R, 3, 5, 5>(L, lane, f0, cur.c0, cur.cend); break;
-        }
-        __syncthreads();
-        // ---- 3. node-owned combine -----------------------------------------
-        if constexpr (NW == 4) {
-            switch (wave) {
-                case 0: combine<R, 0, 0, 8>(L, acc, r, c, cur.k); break;
-                case 1: combine<R, 1, 0, 6>(L, acc, r, c, cur.k); break;
-                case 2: combine<R, 2, 0, 6>(L, acc, r, c, cur.k); break;
-                default: combine<R, 3, 0, 10>(L, acc, r, c, cur.k); break;
-            }
-        } else switch (wave) {
-            case 0: combine<R, 0, 0, 4>(L, acc, r, c, cur.k); break;
-            case 1: combine<R, 1, 0, 3>(L, acc, r, c, cur.k); break;
-            case 2: combine<R, 2, 0, 3>(L, acc, r, c, cur.k); break;
-            case 3: combine<R, 3, 0, 5>(L, acc, r, c, cur.k); break;
-            case 4: combine<R, 0, 4, 4>(L, acc, r, c, cur.k); break;
-            case 5: combine<R, 1, 3, 3>(L, acc, r, c, cur.k); break;
-            case 6: combine<R, 2, 3, 3>(L, acc, r, c, cur.k); break;
-            default: combine<R, 3, 5, 5>(L, acc, r, c, cur.k); break;
-        }
-        // ---- 4. stage the next chunk (the staged values of this one are no
-        // longer read) ---------------------------------------------------------
-        if (nx.k < TILE && ts < nx.cend - nx.c0) {
-#pragma unroll
-            for (int q = 0; q < NSET; ++q) stage_raw(A, L, part + q, ts, raw[q], j0, i0);
-        }
-        __syncthreads();
-        cur = nx;
-        nx = nx2;
-    }
-    if constexpr (NW == 4) {
-        switch (wave) {
-            case 0: write_part<R, 0, 0, 8>(A.part, tile, acc, lane); break;
-            case 1: write_part<R, 1, 0, 6>(A.part, tile, acc, lane); break;
-            case 2: write_part<R, 2, 0, 6>(A.part, tile, acc, lane); break;
-            default: write_part<R, 3, 0, 10>(A.part, tile, acc, lane); break;
-        }
-        return;
-    }
-    switch (wave) {
-        case 0: write_part<R, 0, 0, 4>(A.part, tile, acc, lane); break;
-        case 1: write_part<R, 1, 0, 3>(A.part, tile, acc, lane); break;
-        case 2: write_part<R, 2, 0, 3>(A.part, tile, acc, lane); break;
-        case 3: write_part<R, 3, 0, 5>(A.part, tile, acc, lane); break;
-        case 4: write_part<R, 0, 4, 4>(A.part, tile, acc, lane); break;
-        case 5: write_part<R, 1, 3, 3>(A.part, tile, acc, lane); break;
-        case 6: write_part<R, 2, 3, 3>(A.part, tile, acc, lane); break;
-        default: write_part<R, 3, 5, 5>(A.part, tile, acc, lane); break;
-    }
+    window_sums<TYPED>(L, A.part + (size_t)tile * NSUM * 64, wave, lane);
 }
 
 struct SumPtrs {
@@ -646,18 +741,18 @@ static int launch_scatter_t(ereb_ctx* c) {
         const int rc = typed_refresh(c);
         if (rc) return rc;
     }
-    A.typed = c->typed == 1 ? 1 : 0;
     A.tm = tm_ptr(c);
     A.tab = typed_tab(c->mat);
+    A.typed = c->typed == 1 && tab_finite<R>(A.tab) ? 1 : 0;
     hipEvent_t ev;
     prof_begin(c, EREB_K_SCATTER, &ev);
     // the scatter's completion as ev_scatter when asked (rec_scatter)
-    const dim3 grid((unsigned)c->ntiles), block(ScatterShape<R>::NW * 64);
+    const dim3 grid((unsigned)c->ntiles), block(SCAT_NW * 64);
+    auto* kern = A.typed ? k_scatter<R, true> : k_scatter<R, false>;
     if (c->rec_scatter)
-        hipExtLaunchKernelGGL(k_scatter<R>, grid, block, 0, c->stream, nullptr, c->ev_scatter, 0,
-                              A);
+        hipExtLaunchKernelGGL(kern, grid, block, 0, c->stream, nullptr, c->ev_scatter, 0, A);
     else
-        hipLaunchKernelGGL(k_scatter<R>, grid, block, 0, c->stream, A);
+        hipLaunchKernelGGL(kern, grid, block, 0, c->stream, A);
     c->rec_scatter = false;
     EREB_HIP(c, hipGetLastError());
     prof_end(c, EREB_K_SCATTER, ev);

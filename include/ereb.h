@@ -49,8 +49,8 @@ extern "C" {
 
 /* ---- precision forms --------------------------------------------------- */
 #define EREB_FP64   0  /* every operation in Float64, as the reference */
-#define EREB_MIXED  1  /* properties, weights and interpolation in FP32 with
-                          compensated accumulation; coordinates, RK4 updates,
+#define EREB_MIXED  1  /* properties and stress interpolation in FP32;
+                          coordinates, scatter weights and sums, RK4 updates,
                           node normalisation and matrix coefficients FP64 */
 
 /* ---- geometry: the compile-time constants of C:14-101 ------------------- */
