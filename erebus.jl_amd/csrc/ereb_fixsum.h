@@ -49,16 +49,10 @@ __device__ __forceinline__ bool fix_split(double v, double up, unsigned long lon
     return true;
 }
 
-// PASS 0: record |v| in maxbits.  PASS 1: add v to node k.  `flag` is set
-// when a contribution lies outside the range of the scale (or is not
-// finite), which the host reports as an error.
-template <int PASS>
+// add v to node k.  `flag` is set when a contribution lies outside the range
+// of the scale (or is not finite), which the host reports as an error.
 __device__ __forceinline__ void fix_add(const FixGrid& F, int64_t k, double v, int* flag) {
     if (!F.w || v == 0.0) return;
-    if (PASS == 0) {
-        atomicMax(F.maxbits, (unsigned long long)__double_as_longlong(fabs(v)));
-        return;
-    }
     unsigned long long H, L;
     if (!fix_split(v, F.up, H, L)) {
         atomicOr(flag, 1);

@@ -576,10 +576,10 @@ __device__ void block_fix_add(const FixGrid& F, int rows, bool on, const int (&i
             for (int q = 0; q < NS; ++q) {
                 if (vs[q] == 0.0) continue;
                 const int64_t k = (int64_t)(js[q] - 1) * rows + (is[q] - 1);
-                fix_add<1>(F, k, ws[q][0] * vs[q], flag);
-                fix_add<1>(F, k + 1, ws[q][1] * vs[q], flag);
-                fix_add<1>(F, k + rows, ws[q][2] * vs[q], flag);
-                fix_add<1>(F, k + rows + 1, ws[q][3] * vs[q], flag);
+                fix_add(F, k, ws[q][0] * vs[q], flag);
+                fix_add(F, k + 1, ws[q][1] * vs[q], flag);
+                fix_add(F, k + rows, ws[q][2] * vs[q], flag);
+                fix_add(F, k + rows + 1, ws[q][3] * vs[q], flag);
             }
         }
         return;
