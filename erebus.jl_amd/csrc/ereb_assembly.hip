@@ -330,38 +330,80 @@ __host__ __device__ __forceinline__ void stokes_eq(const AsmArgs& A, int e, int 
     }
 }
 
-// 1. rows: thread per P cell, blockIdx.y = equation (wave-uniform)
-template <int SYS>
+// One system's buffers on the device, and the blocks of its column kernels
+struct AsmSys {
+    const SlotTables* T;
+    uint16_t* pres;      // presence bits of each row's slots
+    double* slotv;
+    uint16_t* prev;      // of the previous assembly (optional)
+    int32_t* chg;        // raised where they differ (optional)
+    int32_t* bsum;       // entries per block of columns
+    int32_t* colptr;
+    int32_t* rowval;
+    double* nzval;
+    int32_t* map;
+    double* R;
+    int64_t n;           // columns
+};
+
+// 1. rows: thread per P cell, equation e (wave-uniform; 0..5 Stokes-Darcy).
 // prev, chg (optional): the presence bits of the previous assembly; where
 // they differ, prev is updated and chg[0] set to 1 (every writer stores the
 // same value), so chg[0] tells whether the pattern changed
-__global__ __launch_bounds__(256) void k_asm_rows(AsmArgs A0, const StepScalars* __restrict__ S,
-                                                  const SlotTables* __restrict__ T,
-                                                  uint16_t* __restrict__ pres_out,
-                                                  double* __restrict__ slotv,
-                                                  int32_t* __restrict__ flags,
-                                                  uint16_t* __restrict__ prev,
-                                                  int32_t* __restrict__ chg) {
+template <int SYS>
+__device__ __forceinline__ void asm_row(const AsmArgs& A0, const StepScalars* __restrict__ S,
+                                        const AsmSys& s, int e, int32_t* __restrict__ flags) {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= A0.Nx1 * A0.Ny1) return;
     AsmArgs A = A0;
     A.dt = S->dt;  // the step's dt from the device block
-    const int e = blockIdx.y;
+    A.R = s.R;
     const int i = k % A.Ny1 + 1, j = k / A.Ny1 + 1;
     const int64_t ncell = (int64_t)A.Nx1 * A.Ny1;
     uint32_t pres = 0;
-    SlotSink sink{T, slotv + (size_t)T->slot0[e] * ncell + k, ncell, &pres, flags, e,
+    SlotSink sink{s.T, s.slotv + (size_t)s.T->slot0[e] * ncell + k, ncell, &pres, flags, e,
                   SYS == 0 ? 6 : 1, A.Ny1};
     if (SYS == 0)
         stokes_eq(A, e, i, j, sink, true);
     else
         thermal_cell(A, i, j, sink, true);
     const size_t q = (size_t)e * ncell + k;
-    pres_out[q] = (uint16_t)pres;
-    if (prev && prev[q] != (uint16_t)pres) {
-        prev[q] = (uint16_t)pres;
-        chg[0] = 1;
+    s.pres[q] = (uint16_t)pres;
+    if (s.prev && s.prev[q] != (uint16_t)pres) {
+        s.prev[q] = (uint16_t)pres;
+        s.chg[0] = 1;
     }
+}
+
+// one system, blockIdx.y = equation
+template <int SYS>
+__global__ __launch_bounds__(256) void k_asm_rows(AsmArgs A, const StepScalars* __restrict__ S,
+                                                  AsmSys s, int32_t* __restrict__ flags) {
+    asm_row<SYS>(A, S, s, blockIdx.y, flags);
+}
+
+// both systems of a step in one launch: blockIdx.y 6 is the thermal equation.
+// The thermal system's kernels are too small to fill the chip and mostly cost
+// their launches (20 us of a 2.8M-marker step one after the other; beside the
+// Stokes-Darcy ones they cost 3, and a step has four launches fewer).
+__global__ __launch_bounds__(256) void k_asm_rows_both(AsmArgs A,
+                                                       const StepScalars* __restrict__ S,
+                                                       AsmSys sd, AsmSys th,
+                                                       int32_t* __restrict__ flags) {
+    if (blockIdx.y < 6) asm_row<0>(A, S, sd, blockIdx.y, flags);
+    else asm_row<1>(A, S, th, 0, flags);
+}
+
+// Two systems' column kernels in one launch: blocks [0, nb0) work on s[0], the
+// others on s[1] (a single system: every block on s[0]).
+struct AsmPair {
+    AsmSys s[2];
+    int nb0;
+};
+__device__ __forceinline__ int pair_block(const AsmPair& P, const AsmSys*& s) {
+    const int second = (int)blockIdx.x >= P.nb0 ? 1 : 0;
+    s = &P.s[second];
+    return (int)blockIdx.x - (second ? P.nb0 : 0);
 }
 
 // 2. column counts per block of columns: one thread per column walks the
@@ -400,12 +442,13 @@ __device__ __forceinline__ int32_t asm_block_scan(int32_t v, int32_t* sh, int32_
     return r;
 }
 
-__global__ __launch_bounds__(256) void k_asm_count(int Nx1, int Ny1,
-                                                   const SlotTables* __restrict__ Tg,
-                                                   const uint16_t* __restrict__ pres,
-                                                   int32_t* __restrict__ bsum,
-                                                   const int32_t* __restrict__ run) {
-    if (run && run[0] == 0) return;
+__global__ __launch_bounds__(256) void k_asm_count(int Nx1, int Ny1, AsmPair P) {
+    const AsmSys* s;
+    const int blk = pair_block(P, s);
+    if (s->chg && s->chg[0] == 0) return;
+    const SlotTables* __restrict__ Tg = s->T;
+    const uint16_t* __restrict__ pres = s->pres;
+    int32_t* __restrict__ bsum = s->bsum;
     __shared__ SlotTables T;
     __shared__ int32_t sh[17];
     static_assert(sizeof(SlotTables) % 4 == 0, "table size");
@@ -414,7 +457,7 @@ __global__ __launch_bounds__(256) void k_asm_count(int Nx1, int Ny1,
     __syncthreads();
     const int ne = T.ne;
     const int64_t ncell = (int64_t)Nx1 * Ny1;
-    const int64_t col = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t col = (int64_t)blk * blockDim.x + threadIdx.x;
     int32_t p = 0;
     if (col < ncell * ne) {
         const int u = (int)(col % ne);
@@ -431,7 +474,7 @@ __global__ __launch_bounds__(256) void k_asm_count(int Nx1, int Ny1,
     }
     int32_t tot;
     asm_block_scan(p, sh, &tot);
-    if (threadIdx.x == 0) bsum[blockIdx.x] = tot;
+    if (threadIdx.x == 0) bsum[blk] = tot;
 }
 
 // 3. colptr/rowval/nzval: the same column walk; a column's start is the sum
@@ -454,20 +497,18 @@ constexpr int ASM_STAGE = 4096;
 // loads, and half the LDS: twice the workgroups per CU).
 // IDX, BASE: the row index type and base of the output (int32 0-based for
 // the context's device CSC, Int64 1-based for SparseMatrixCSC{Float64,Int64})
-// run (optional): only when run[0] != 0; map (optional): the slot value's
-// index of every stored entry, for the values-only refill
+// map (optional): the slot value's index of every stored entry, for the
+// values-only refill
 template <int MAXR, class IDX = int32_t, int BASE = 0, bool VALUES = false>
-__global__ __launch_bounds__(256) void k_asm_fill(int Nx1, int Ny1,
-                                                  const SlotTables* __restrict__ Tg,
-                                                  const uint16_t* __restrict__ pres,
-                                                  const double* __restrict__ slotv,
-                                                  const int32_t* __restrict__ bsum,
-                                                  int32_t* __restrict__ colptr,
-                                                  IDX* __restrict__ rowval,
-                                                  double* __restrict__ nzval,
-                                                  const int32_t* __restrict__ run,
-                                                  int32_t* __restrict__ map) {
-    if (run && run[0] == 0) return;
+__device__ __forceinline__ void asm_fill(int Nx1, int Ny1, const AsmSys& s, int blk,
+                                         IDX* __restrict__ rowval) {
+    const SlotTables* __restrict__ Tg = s.T;
+    const uint16_t* __restrict__ pres = s.pres;
+    const double* __restrict__ slotv = s.slotv;
+    const int32_t* __restrict__ bsum = s.bsum;
+    int32_t* __restrict__ colptr = s.colptr;
+    double* __restrict__ nzval = s.nzval;
+    int32_t* __restrict__ map = s.map;
     __shared__ SlotTables T;
     __shared__ int32_t srow[ASM_STAGE];
     __shared__ int32_t smap[ASM_STAGE];
@@ -477,12 +518,12 @@ __global__ __launch_bounds__(256) void k_asm_fill(int Nx1, int Ny1,
         ((int32_t*)&T)[q] = ((const int32_t*)Tg)[q];
     // entries of the blocks before this one
     int32_t before = 0;
-    for (int b = threadIdx.x; b < (int)blockIdx.x; b += blockDim.x) before += bsum[b];
+    for (int b = threadIdx.x; b < blk; b += blockDim.x) before += bsum[b];
     int32_t base;
     asm_block_scan(before, sh, &base);  // synchronises: T is staged
     const int ne = T.ne;
     const int64_t ncell = (int64_t)Nx1 * Ny1, n = ncell * ne;
-    const int64_t col0 = (int64_t)blockIdx.x * blockDim.x;
+    const int64_t col0 = (int64_t)blk * blockDim.x;
     const int64_t col = col0 + threadIdx.x;
     bool on[MAXR];
     int32_t rw[MAXR], mp[MAXR];
@@ -533,6 +574,19 @@ __global__ __launch_bounds__(256) void k_asm_fill(int Nx1, int Ny1,
     }
 }
 
+template <int MAXR>
+__global__ __launch_bounds__(256) void k_asm_fill(int Nx1, int Ny1, AsmPair P) {
+    const AsmSys* s;
+    const int blk = pair_block(P, s);
+    if (s->chg && s->chg[0] == 0) return;
+    asm_fill<MAXR>(Nx1, Ny1, *s, blk, s->rowval);
+}
+// with nzval, into caller buffers with 1-based Int64 rows
+__global__ __launch_bounds__(256) void k_asm_fill_1based(int Nx1, int Ny1, AsmSys s,
+                                                         int64_t* __restrict__ rowval) {
+    asm_fill<16, int64_t, 1, true>(Nx1, Ny1, s, (int)blockIdx.x, rowval);
+}
+
 // nzval through the stored slot indices (after every fill, and alone while
 // the pattern is unchanged): one coalesced write, one gather per entry, in a
 // grid-stride loop over the entries (nnz is known on the device only) with
@@ -541,15 +595,17 @@ __global__ __launch_bounds__(256) void k_asm_fill(int Nx1, int Ny1,
 // for the next assembly's rows kernel.
 constexpr int ASM_VALUES_PER = 4;
 constexpr int ASM_VALUES_BLOCKS = 8192;
-__global__ __launch_bounds__(256) void k_asm_values(const int32_t* __restrict__ colptr_end,
-                                                    const int32_t* __restrict__ map,
-                                                    const double* __restrict__ slotv,
-                                                    double* __restrict__ nzval,
-                                                    int32_t* __restrict__ chg) {
-    if (chg && blockIdx.x == 0 && threadIdx.x == 0) chg[0] = 0;
-    const int64_t nnz = colptr_end[0];
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t q0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q0 < nnz;
+__global__ __launch_bounds__(256) void k_asm_values(AsmPair P) {
+    const AsmSys* s;
+    const int blk = pair_block(P, s);
+    const int nblk = s == &P.s[0] ? P.nb0 : (int)gridDim.x - P.nb0;
+    if (s->chg && blk == 0 && threadIdx.x == 0) s->chg[0] = 0;
+    const int32_t* __restrict__ map = s->map;
+    const double* __restrict__ slotv = s->slotv;
+    double* __restrict__ nzval = s->nzval;
+    const int64_t nnz = s->colptr[s->n];
+    const int64_t stride = (int64_t)nblk * blockDim.x;
+    for (int64_t q0 = (int64_t)blk * blockDim.x + threadIdx.x; q0 < nnz;
          q0 += ASM_VALUES_PER * stride) {
         int32_t mi[ASM_VALUES_PER];
         double v[ASM_VALUES_PER];
@@ -675,8 +731,8 @@ int host_slot_check(int64_t* slots_sd, int64_t* slots_t) {
     return EREB_OK;
 }
 
-static AsmArgs asm_args(ereb_ctx* c, double dt, Sys& s) {
-    AsmArgs A;
+static AsmArgs asm_args(ereb_ctx* c, double dt) {
+    AsmArgs A{};
     A.Nx = c->Nx;
     A.Ny = c->Ny;
     A.Nx1 = c->Nx1;
@@ -701,12 +757,12 @@ static AsmArgs asm_args(ereb_ctx* c, double dt, Sys& s) {
     A.tk1 = gptr(c, EREB_G_TK1); A.RHOCP = gptr(c, EREB_G_RHOCP); A.KX = gptr(c, EREB_G_KX);
     A.KY = gptr(c, EREB_G_KY); A.HR = gptr(c, EREB_G_HR); A.HA = gptr(c, EREB_G_HA);
     A.HS = gptr(c, EREB_G_HS); A.DHP = gptr(c, EREB_G_DHP);
-    A.R = s.rhs;
     return A;
 }
 
+// one system's tables and buffers ready, its AsmSys
 template <int SYS>
-static int assemble(ereb_ctx* c, double dt) {
+static int sys_ready(ereb_ctx* c, AsmSys& K) {
     Sys& s = c->sys[SYS];
     if (!s.tables) {
         SlotTables T;
@@ -720,50 +776,68 @@ static int assemble(ereb_ctx* c, double dt) {
         for (int u = 0; u < T.ne; ++u) s.maxrev = std::max(s.maxrev, T.nrev[u]);
     }
     const int64_t ncell = (int64_t)c->Nx1 * c->Ny1;
-    const int64_t n = ncell * s.ne;
-    const int64_t cap = ncell * s.nstot;  // every slot present
-    int rc = ensure_sys(c, SYS, n, cap, ncell);
+    int rc = ensure_sys(c, SYS, ncell * s.ne, ncell * s.nstot, ncell);  // every slot present
     if (rc) return rc;
-    if ((rc = set_dt(c, dt))) return rc;
-    AsmArgs A = asm_args(c, dt, s);
-    const SlotTables* T = (const SlotTables*)s.tables;
-    hipEvent_t ev;
-    prof_begin(c, SYS == 0 ? EREB_K_ASM_SD : EREB_K_ASM_T, &ev);
-    // pattern unchanged since the previous assembly?  The rows kernel compares
-    // the presence bits as it writes them and raises the flag, which the
-    // values kernel clears at the end of every assembly; with no previous
-    // assembly (a fresh system) it is raised here.
-    if (!s.have_prev && (rc = fill_i32(c, s.chg, 1, 1))) return rc;
-    const dim3 grid((unsigned)((ncell + 255) / 256), (unsigned)s.ne);
-    hipLaunchKernelGGL(k_asm_rows<SYS>, grid, dim3(256), 0, c->stream, A, c->d_scal, T, s.pres,
-                       s.slotv, c->d_flags, s.pres_prev, s.chg);
+    K = AsmSys{(const SlotTables*)s.tables, s.pres, s.slotv, s.pres_prev, s.chg, s.colcnt,
+               s.colptr, s.rowval, s.nzval, s.map, s.rhs, s.n};
+    return EREB_OK;
+}
+
+// pattern unchanged since the previous assembly?  The rows kernel compares
+// the presence bits as it writes them and raises the flag, which the
+// values kernel clears at the end of every assembly; with no previous
+// assembly (a fresh system) it is raised here.
+static int sys_fresh(ereb_ctx* c, Sys& s) {
+    const int rc = s.have_prev ? EREB_OK : fill_i32(c, s.chg, 1, 1);
     s.have_prev = true;
-    const int32_t* chg = s.chg;
+    return rc;
+}
+
+// count, fill and values of one or two systems (K1 null: one)
+static int launch_columns(ereb_ctx* c, const AsmSys& K0, const Sys& s0, const AsmSys* K1,
+                          const Sys* s1) {
     // a block's entries must fit the LDS stage: 256 columns of up to 16
     // entries, else 128 of up to 32 (SLOT_R); the count's blocks are the
     // fill's
-    const bool narrow = s.maxrev <= ASM_STAGE / 256;
+    const bool narrow = s0.maxrev <= ASM_STAGE / 256 && (!s1 || s1->maxrev <= ASM_STAGE / 256);
     static_assert(ASM_STAGE / 256 == 16, "16 candidates per column in the 256-column blocks");
     static_assert(ASM_STAGE / 128 >= SLOT_R, "stage holds 128 columns of SLOT_R entries");
     const int fb = narrow ? 256 : 128;
-    const dim3 fgrid((unsigned)((n + fb - 1) / fb));
-    hipLaunchKernelGGL(k_asm_count, fgrid, dim3(fb), 0, c->stream, c->Nx1, c->Ny1, T, s.pres,
-                       s.colcnt, chg);
+    auto cols = [&](const Sys& s) { return (unsigned)((s.n + fb - 1) / fb); };
+    auto vals = [&](const Sys& s) {
+        return (unsigned)std::min<int64_t>(
+            (s.cap + 256 * ASM_VALUES_PER - 1) / (256 * ASM_VALUES_PER), ASM_VALUES_BLOCKS);
+    };
+    AsmPair P{{K0, K1 ? *K1 : K0}, (int)cols(s0)};
+    const dim3 fgrid(cols(s0) + (s1 ? cols(*s1) : 0));
+    hipLaunchKernelGGL(k_asm_count, fgrid, dim3(fb), 0, c->stream, c->Nx1, c->Ny1, P);
     if (narrow)
-        hipLaunchKernelGGL(k_asm_fill<16>, fgrid, dim3(fb), 0, c->stream, c->Nx1, c->Ny1, T,
-                           s.pres, s.slotv, (const int32_t*)s.colcnt, s.colptr, s.rowval,
-                           s.nzval, chg, s.map);
+        hipLaunchKernelGGL(k_asm_fill<16>, fgrid, dim3(fb), 0, c->stream, c->Nx1, c->Ny1, P);
     else
-        hipLaunchKernelGGL(k_asm_fill<SLOT_R>, fgrid, dim3(fb), 0, c->stream, c->Nx1, c->Ny1, T,
-                           s.pres, s.slotv, (const int32_t*)s.colcnt, s.colptr, s.rowval,
-                           s.nzval, chg, s.map);
-    hipLaunchKernelGGL(k_asm_values,
-                       dim3((unsigned)std::min<int64_t>(
-                           (cap + 256 * ASM_VALUES_PER - 1) / (256 * ASM_VALUES_PER),
-                           ASM_VALUES_BLOCKS)),
-                       dim3(256), 0, c->stream, (const int32_t*)s.colptr + n,
-                       (const int32_t*)s.map, (const double*)s.slotv, s.nzval, s.chg);
+        hipLaunchKernelGGL(k_asm_fill<SLOT_R>, fgrid, dim3(fb), 0, c->stream, c->Nx1, c->Ny1, P);
+    P.nb0 = (int)vals(s0);
+    hipLaunchKernelGGL(k_asm_values, dim3(vals(s0) + (s1 ? vals(*s1) : 0)), dim3(256), 0,
+                       c->stream, P);
     EREB_HIP(c, hipGetLastError());
+    return EREB_OK;
+}
+
+static unsigned cell_blocks(const ereb_ctx* c) {
+    return (unsigned)(((int64_t)c->Nx1 * c->Ny1 + 255) / 256);
+}
+
+template <int SYS>
+static int assemble(ereb_ctx* c, double dt) {
+    AsmSys K;
+    int rc = sys_ready<SYS>(c, K);
+    if (rc || (rc = set_dt(c, dt))) return rc;
+    Sys& s = c->sys[SYS];
+    hipEvent_t ev;
+    prof_begin(c, SYS == 0 ? EREB_K_ASM_SD : EREB_K_ASM_T, &ev);
+    if ((rc = sys_fresh(c, s))) return rc;
+    hipLaunchKernelGGL(k_asm_rows<SYS>, dim3(cell_blocks(c), (unsigned)s.ne), dim3(256), 0,
+                       c->stream, asm_args(c, dt), c->d_scal, K, c->d_flags);
+    if ((rc = launch_columns(c, K, s, nullptr, nullptr))) return rc;
     prof_end(c, SYS == 0 ? EREB_K_ASM_SD : EREB_K_ASM_T, ev);
     s.valid = true;
     return EREB_OK;
@@ -771,6 +845,24 @@ static int assemble(ereb_ctx* c, double dt) {
 
 int launch_assemble_stokes(ereb_ctx* c, double dt) { return assemble<0>(c, dt); }
 int launch_assemble_thermal(ereb_ctx* c, double dt) { return assemble<1>(c, dt); }
+
+int launch_assemble_both(ereb_ctx* c, double dt) {
+    int rc;
+    if (c->prof) {  // timed as two classes
+        if ((rc = assemble<0>(c, dt))) return rc;
+        return assemble<1>(c, dt);
+    }
+    AsmSys K0, K1;
+    if ((rc = sys_ready<0>(c, K0)) || (rc = sys_ready<1>(c, K1)) || (rc = set_dt(c, dt)))
+        return rc;
+    Sys &s0 = c->sys[0], &s1 = c->sys[1];
+    if ((rc = sys_fresh(c, s0)) || (rc = sys_fresh(c, s1))) return rc;
+    hipLaunchKernelGGL(k_asm_rows_both, dim3(cell_blocks(c), 7), dim3(256), 0, c->stream,
+                       asm_args(c, dt), c->d_scal, K0, K1, c->d_flags);
+    if ((rc = launch_columns(c, K0, s0, &K1, &s1))) return rc;
+    s0.valid = s1.valid = true;
+    return EREB_OK;
+}
 
 // ---- thermal assembly into caller buffers, scratch supplied ------------------
 // Scratch layout (each piece 256-byte aligned): the step scalars (dt), the
@@ -848,18 +940,22 @@ int launch_thermal_noalloc(ereb_ctx* c, char* scratch, const double* const in[8]
     A.HA = in[5];
     A.HS = in[6];
     A.DHP = in[7];
-    A.R = RT;
     const dim3 grid((unsigned)((ncell + 255) / 256), 1);
+    AsmSys K{};
+    K.T = t.tables;
+    K.pres = t.pres;
+    K.slotv = t.slotv;
+    K.bsum = t.colcnt;
+    K.colptr = t.colptr;
+    K.nzval = nzval;
+    K.R = RT;
+    K.n = ncell;
     hipLaunchKernelGGL(k_asm_rows<1>, grid, dim3(256), 0, c->stream, A,
-                       (const StepScalars*)t.scal, (const SlotTables*)t.tables, t.pres, t.slotv,
-                       t.flags, (uint16_t*)nullptr, (int32_t*)nullptr);
+                       (const StepScalars*)t.scal, K, t.flags);
     hipLaunchKernelGGL(k_asm_count, grid, dim3(256), 0, c->stream, c->Nx1, c->Ny1,
-                       (const SlotTables*)t.tables, (const uint16_t*)t.pres, t.colcnt,
-                       (const int32_t*)nullptr);
-    hipLaunchKernelGGL((k_asm_fill<16, int64_t, 1, true>), grid, dim3(256), 0, c->stream, c->Nx1,
-                       c->Ny1, (const SlotTables*)t.tables, (const uint16_t*)t.pres,
-                       (const double*)t.slotv, (const int32_t*)t.colcnt, t.colptr, rowval,
-                       nzval, (const int32_t*)nullptr, (int32_t*)nullptr);
+                       AsmPair{{K, K}, (int)grid.x});
+    hipLaunchKernelGGL(k_asm_fill_1based, grid, dim3(256), 0, c->stream, c->Nx1, c->Ny1, K,
+                       rowval);
     hipLaunchKernelGGL(k_colptr_1based, dim3((unsigned)((ncell + 1 + 255) / 256)), dim3(256), 0,
                        c->stream, (const int32_t*)t.colptr, colptr, ncell + 1);
     EREB_HIP(c, hipGetLastError());

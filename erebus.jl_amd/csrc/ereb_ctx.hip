@@ -343,9 +343,8 @@ int ereb_ctx_create(const ereb_geometry* g, const ereb_materials* mat, int preci
         std::vector<uint32_t> all((size_t)(prop.multiProcessorCount + 31) / 32, ~0u);
         CK(hipExtStreamCreateWithCUMask(&c->stream2, (uint32_t)all.size(), all.data()));
     }
-    // recorded as kernels' stop events (hipExtLaunchKernelGGL): default flags
+    // recorded as a kernel's stop event (hipExtLaunchKernelGGL): default flags
     CK(hipEventCreate(&c->ev_scatter));
-    CK(hipEventCreate(&c->ev_keys));
     CK(hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming));
     // the no-alloc entry point's scratch on this device (once per device); a
     // failure here is reported by that entry point, which tries again
@@ -392,7 +391,6 @@ int ereb_ctx_create(const ereb_geometry* g, const ereb_materials* mat, int preci
     // the sort leaves the key counts at zero for the next sort
     CK(hipMemset(c->d_fcount, 0, sizeof(int32_t) * c->nkeys));
     CK(hipMalloc(&c->d_fstart, sizeof(int32_t) * (c->nkeys + 1)));
-    CK(hipMalloc(&c->d_big, sizeof(int32_t) * (c->nkeys + 1)));
     CK(hipMalloc(&c->d_flags, sizeof(int32_t) * 4));
     CK(hipMemset(c->d_flags, 0, sizeof(int32_t) * 4));
     CK(hipMalloc(&c->d_part, sizeof(double) * (size_t)c->ntiles * NSUM * 64));
@@ -429,7 +427,6 @@ int ereb_ctx_destroy(ereb_ctx* c) {
     hipFree(c->d_tmp);
     hipFree(c->d_fcount);
     hipFree(c->d_fstart);
-    hipFree(c->d_big);
     hipFree(c->d_flags);
     hipFree(c->d_part);
     hipFree(c->d_typed);
@@ -451,7 +448,7 @@ int ereb_ctx_destroy(ereb_ctx* c) {
         hipFree(s.chg);
         hipFree(s.map);
     }
-    for (hipEvent_t e : {c->ev_scatter, c->ev_join, c->ev_keys})
+    for (hipEvent_t e : {c->ev_scatter, c->ev_join})
         if (e) hipEventDestroy(e);
     if (c->stream2) hipStreamDestroy(c->stream2);
     if (c->stream) hipStreamDestroy(c->stream);
@@ -636,32 +633,42 @@ struct OnStream {
     ~OnStream() { c->stream = s0; }
 };
 
-// The step in four segments on two streams.  The stress and temperature
+// The step in three segments on two streams.  The stress and temperature
 // gathers and RK4 (one pass over the markers) read the velocity, rotation,
 // stress-change and temperature grids given to the step, which no kernel of
 // the step writes, and write marker state that the sort and the scatter read;
 // the node pass and the two assemblies read the scatter's window sums and
 // node grids only.  So the marker pass (SEG_MARKERS) runs on the second
-// stream as soon as the scatter (SEG_SCATTER) is done, beside the node pass
-// and the assemblies (SEG_NODES), and its coefficient tables (SEG_TABLES,
-// from the velocities alone) before it, from the end of the sort's key pass
-// (beside the key pass itself, which is bound by HBM traffic, they stretched
-// it by more than their own duration); the main stream waits for the second
-// at the end.  Results are those of the launches in sequence: no kernel of
-// one stream touches what the other's write.
-enum { SEG_TABLES = 0, SEG_SCATTER, SEG_MARKERS, SEG_NODES };
+// stream as soon as the scatter (SEG_SCATTER, whose sort also fills the
+// marker pass's coefficient tables) is done, beside the node pass and the
+// assemblies (SEG_NODES); the main stream waits for the second at the end.
+// Results are those of the launches in sequence: no kernel of one stream
+// touches what the other's write.
+enum { SEG_SCATTER = 0, SEG_MARKERS, SEG_NODES };
+
+// Steps of at most this many markers run in sequence on the main stream.  The
+// second stream's event calls cost the host ~43 us a step, as much as all of
+// its 12 launches, and the marker pass that it hides is short.  us per step, one
+// stream / two: a context by itself 73 / 88 at 3,136 markers, 101 / 104 at
+// 160,000, 131 / 128 at 313,600, 216 / 198 at 1,000,000; three contexts in turn
+// 43 / 90, 45 / 85, 77 / 108, 172 / 199.
+constexpr int64_t ONE_STREAM_MAX = 400000;
 
 static int seg_launches(ereb_ctx* c, int seg, const double* hrs, const double* hrf,
                         int64_t mode, double dt, int64_t timestep) {
     int rc;
     switch (seg) {
-        case SEG_TABLES: return launch_gathers_rk4(c, dt, (int)mode, timestep, RK4_TABLES);
-        case SEG_SCATTER: return launch_scatter(c, hrs, hrf, (int)mode);
-        case SEG_MARKERS: return launch_gathers_rk4(c, dt, (int)mode, timestep, RK4_MARKERS);
+        case SEG_SCATTER:
+            c->tables_ride = c->marknum > 0 && !c->prof;
+            rc = launch_scatter(c, hrs, hrf, (int)mode);
+            c->tables_ride = false;
+            return rc;
+        case SEG_MARKERS:
+            // timed per class: the tables with the marker pass, else beside the sort
+            return launch_gathers_rk4(c, dt, (int)mode, timestep, c->prof);
         default:
             if ((rc = launch_combine_nodes(c))) return rc;
-            if ((rc = launch_assemble_stokes(c, dt))) return rc;
-            return launch_assemble_thermal(c, dt);
+            return launch_assemble_both(c, dt);
     }
 }
 
@@ -680,34 +687,25 @@ static int seg_run(ereb_ctx* c, int seg, hipStream_t s, bool replay, const doubl
 static int transfer_run(ereb_ctx* c, bool replay, const double* hrs, const double* hrf,
                         int64_t mode, double dt, int64_t timestep) {
     int rc;
-    // with per-launch timing on: every launch in sequence on the main stream,
-    // the coefficient tables and the marker pass timed together as one class
-    if (c->prof) {
-        for (int seg : {SEG_SCATTER, SEG_NODES})
+    // with per-launch timing on, and for few markers: every launch in sequence
+    // on the main stream
+    if (c->prof || (!replay && c->marknum <= ONE_STREAM_MAX)) {
+        for (int seg : {SEG_SCATTER, SEG_NODES, SEG_MARKERS})
             if ((rc = seg_launches(c, seg, hrs, hrf, mode, dt, timestep))) return rc;
-        return launch_gathers_rk4(c, dt, (int)mode, timestep);
+        return EREB_OK;
     }
     hipStream_t s1 = c->stream, s2 = c->stream2;
-    // eager: the coefficient tables start once the sort's key pass is done,
-    // beside the rest of the sort (short launches that leave most of the
-    // chip idle); a replay runs them after the scatter (a segment graph
-    // holds no event)
-    // (the key pass and the scatter record their events themselves, as
-    // their completion; a replay records the scatter's after its graph)
-    const bool evs = !replay && c->marknum > 0;
-    c->rec_keys = c->rec_scatter = evs;
+    // eager: the scatter records its event itself, as its completion; a
+    // replay records it after its graph
+    c->rec_scatter = !replay && c->marknum > 0;
+    const bool asked = c->rec_scatter;
     rc = seg_run(c, SEG_SCATTER, s1, replay, hrs, hrf, mode, dt, timestep);
-    const bool keys = evs && !c->rec_keys, scattered = evs && !c->rec_scatter;
-    c->rec_keys = c->rec_scatter = false;
-    if (!rc && keys) {
-        EREB_HIP(c, hipStreamWaitEvent(s2, c->ev_keys, 0));
-        rc = seg_run(c, SEG_TABLES, s2, replay, hrs, hrf, mode, dt, timestep);
-    }
+    const bool scattered = asked && !c->rec_scatter;
+    c->rec_scatter = false;
     if (!rc) {
         if (!scattered) EREB_HIP(c, hipEventRecord(c->ev_scatter, s1));
         EREB_HIP(c, hipStreamWaitEvent(s2, c->ev_scatter, 0));
-        if (!keys) rc = seg_run(c, SEG_TABLES, s2, replay, hrs, hrf, mode, dt, timestep);
-        if (!rc) rc = seg_run(c, SEG_MARKERS, s2, replay, hrs, hrf, mode, dt, timestep);
+        rc = seg_run(c, SEG_MARKERS, s2, replay, hrs, hrf, mode, dt, timestep);
     }
     if (!rc) rc = seg_run(c, SEG_NODES, s1, replay, hrs, hrf, mode, dt, timestep);
     // the join also after a failure: later work on the main stream follows

@@ -29,10 +29,11 @@ struct GeomK {
 // run of the grid, so neighbouring workgroups (neighbouring tiles, runs of
 // markers) share one L2 and the lines straddling their data are fetched
 // once.  A bijection of [0, gridDim.x).
-__device__ __forceinline__ uint32_t xcd_block() {
-    const uint32_t nb = gridDim.x, b = blockIdx.x, q = nb >> 3, r = nb & 7, x = b & 7;
+__device__ __forceinline__ uint32_t xcd_block(uint32_t nb, uint32_t b) {
+    const uint32_t q = nb >> 3, r = nb & 7, x = b & 7;
     return x * q + min(x, r) + (b >> 3);
 }
+__device__ __forceinline__ uint32_t xcd_block() { return xcd_block(gridDim.x, blockIdx.x); }
 
 // Node k (1-based) of an axis with spacing h.  EXACT (the context found
 // every node of every axis equal to the first node plus k*h rounded once,

@@ -89,7 +89,7 @@ struct StepKey {
 
 // segments of the transfer step, each captured as a graph of its own
 // (ereb_step_transfer)
-constexpr int NSTEP_SEG = 4;
+constexpr int NSTEP_SEG = 3;
 
 }  // namespace ereb
 
@@ -98,13 +98,16 @@ struct ereb_ctx {
     hipStream_t stream = nullptr;
     // second stream of the transfer step (default priority, like `stream`):
     // the gathers and RK4 run there beside the node pass and the assemblies;
-    // scatter-done, join and key-pass-done events; while rec_keys /
-    // rec_scatter is set, the next key pass / scatter launch records ev_keys /
-    // ev_scatter as its own completion (hipExtLaunchKernelGGL's stop event,
-    // no marker packet between two kernels of the stream) and clears the flag
+    // scatter-done and join events; while rec_scatter is set, the next scatter
+    // launch records ev_scatter as its own completion (hipExtLaunchKernelGGL's
+    // stop event, no marker packet between two kernels of the stream) and
+    // clears the flag
     hipStream_t stream2 = nullptr;
-    hipEvent_t ev_scatter = nullptr, ev_join = nullptr, ev_keys = nullptr;
-    bool rec_keys = false, rec_scatter = false;
+    hipEvent_t ev_scatter = nullptr, ev_join = nullptr;
+    bool rec_scatter = false;
+    // the next sort's placement also fills the RK4 coefficient tables (set by a
+    // transfer step with markers, cleared by the launch)
+    bool tables_ride = false;
     int precision = EREB_FP64;
     int Nx = 0, Ny = 0, Nx1 = 0, Ny1 = 0;
     double dx = 0, dy = 0;
@@ -141,7 +144,6 @@ struct ereb_ctx {
     int64_t tmp_cap = 0;
     int32_t* d_fcount = nullptr;   // nkeys
     int32_t* d_fstart = nullptr;   // nkeys + 1
-    int32_t* d_big = nullptr;      // nkeys + 1: [0] = count, then key ids
     int32_t* d_flags = nullptr;    // [0] domain error
     double* d_part = nullptr;      // ntiles * NSUM * 64
     int32_t* d_scan = nullptr;     // scan block sums
@@ -284,16 +286,16 @@ int launch_gather_stress(ereb_ctx* c);
 // xb_out/yb_out (optional): fluid back-trace end points, for the adjoint
 int launch_rk4(ereb_ctx* c, double dt, int mode, double* xb_out = nullptr,
                double* yb_out = nullptr);
-// stress gather, temperature gather (timestep) and RK4 in one kernel.  parts:
-// RK4_TABLES launches the stage-velocity coefficient tables (they depend on
-// the velocity grids only), RK4_MARKERS the marker kernel, which reads them
-constexpr int RK4_TABLES = 1, RK4_MARKERS = 2;
-int launch_gathers_rk4(ereb_ctx* c, double dt, int mode, int64_t timestep,
-                       int parts = RK4_TABLES | RK4_MARKERS);
+// stress gather, temperature gather (timestep) and RK4 in one kernel; tables:
+// the stage-velocity coefficient tables first (they depend on the velocity
+// grids only), else they are filled already
+int launch_gathers_rk4(ereb_ctx* c, double dt, int mode, int64_t timestep, bool tables);
 
 // ereb_assembly.hip
 int launch_assemble_stokes(ereb_ctx* c, double dt);
 int launch_assemble_thermal(ereb_ctx* c, double dt);
+// both, their kernels sharing launches (apart while profiling)
+int launch_assemble_both(ereb_ctx* c, double dt);
 // Thermal assembly into caller buffers with no allocation: grids in (device
 // pointers, (Ny1, Nx1)), RT and a 1-based Int64 CSC out; `scratch` holds at
 // least thermal_scratch_bytes(ncell) bytes, 256-byte aligned; dt is read

@@ -16,12 +16,15 @@
 //                     properties
 //   2. scan         : key starts
 //   3. k_fine_place : perm[start of the key + rank] = marker, no atomics
+//                     (in the transfer step also the RK4 coefficient tables,
+//                     by workgroups of their own);
 //   4. k_fine_order : each key segment (about 9 markers) is sorted by marker
 //                     index in place (in registers up to 16 markers),
 //                     removing the arrival order of step 3;
-//                     segments longer than SEG_THREAD go to k_fine_order_big
+//                     segments longer than SEG_THREAD by the whole workgroup
 //                     (bitonic in LDS up to 16384, global memory beyond).
 #include "ereb_internal.h"
+#include "ereb_rkcoef.h"
 
 namespace ereb {
 
@@ -92,11 +95,9 @@ __global__ __launch_bounds__(256) void k_fine_count(GeomK g, int nty, const doub
                                                     uint32_t* __restrict__ key,
                                                     int32_t* __restrict__ rank,
                                                     int32_t* __restrict__ count,
-                                                    int32_t* __restrict__ flags,
-                                                    int32_t* __restrict__ big, P props) {
+                                                    int32_t* __restrict__ flags, P props) {
     const int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const bool active = m < M;
-    if (m == 0) big[0] = 0;  // k_fine_order, which fills the list, runs after
     uint32_t k = 0;
     if (active) {
         bool bad;
@@ -139,31 +140,73 @@ static PropArgs<R> prop_args(ereb_ctx* c, const PropsReq& q) {
 // each marker to its sorted slot: the key's start plus its rank.  The
 // workgroups are numbered XCD-contiguously, so that neighbouring marker
 // columns, whose markers fill the same key segments, write through one L2.
+__device__ __forceinline__ void fine_place(int64_t m, const uint32_t* __restrict__ key,
+                                           const int32_t* __restrict__ rank, int64_t M,
+                                           const int32_t* __restrict__ start,
+                                           uint32_t* __restrict__ perm) {
+    if (m < M) perm[start[key[m]] + rank[m]] = (uint32_t)m;
+}
 __global__ __launch_bounds__(256) void k_fine_place(const uint32_t* __restrict__ key,
                                                     const int32_t* __restrict__ rank, int64_t M,
                                                     const int32_t* __restrict__ start,
                                                     uint32_t* __restrict__ perm) {
-    const int64_t m = (int64_t)xcd_block() * blockDim.x + threadIdx.x;
-    if (m < M) perm[start[key[m]] + rank[m]] = (uint32_t)m;
+    fine_place((int64_t)xcd_block() * blockDim.x + threadIdx.x, key, rank, M, start, perm);
+}
+
+// The placement and, in the workgroups from nplace on, the RK4 coefficient
+// tables, which depend on the velocities only: in a launch of their own on the
+// second stream they cost the step a launch and two event calls (~15 us of
+// host time; the step of a 15 x 15 grid is its launches), and take the
+// placement's memory latency here (16 us alone, 18 with the tables at 2.8M
+// markers).
+__global__ __launch_bounds__(256) void k_fine_place_tables(const uint32_t* __restrict__ key,
+                                                           const int32_t* __restrict__ rank,
+                                                           int64_t M,
+                                                           const int32_t* __restrict__ start,
+                                                           uint32_t* __restrict__ perm,
+                                                           uint32_t nplace, uint32_t ntab,
+                                                           RKCoefArgs A) {
+    static_assert(RKCOEF_CELLS == 256, "one workgroup size for both");
+    __shared__ double sh[RKCOEF_CELLS * RKC];
+    if (blockIdx.x < nplace) {
+        fine_place((int64_t)xcd_block(nplace, blockIdx.x) * 256 + threadIdx.x, key, rank, M, start,
+                   perm);
+        return;
+    }
+    const uint32_t b = blockIdx.x - nplace;
+    rk4_coef_block(A, (int)(b % ntab), (int)(b / ntab), sh);
 }
 
 constexpr int SEG_REG = 16;     // segments ordered in registers by rank
 constexpr int SEG_THREAD = 48;  // longest segment ordered by one thread
 constexpr int SEG_BIG = 16384;  // longest segment ordered in LDS (64 KB)
+constexpr int ORD_T = 1024;     // keys per workgroup
 
-__global__ __launch_bounds__(256) void k_fine_order(const int32_t* __restrict__ start, int64_t nkeys,
-                                                    uint32_t* __restrict__ perm,
-                                                    int32_t* __restrict__ big) {
-    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= nkeys) return;
-    const int32_t a = start[k], e = start[k + 1];
-    if (e - a <= 1) return;
+// one thread per key; keys of more than SEG_THREAD markers are then ordered by
+// the whole workgroup, one after the other (a launch of its own for them, with
+// nothing to do in most steps, cost 5 us).  tmp: scratch of 2 M words.
+__global__ __launch_bounds__(ORD_T) void k_fine_order(const int32_t* __restrict__ start,
+                                                      int64_t nkeys, uint32_t* __restrict__ perm,
+                                                      uint32_t* __restrict__ tmp) {
+    extern __shared__ uint32_t sdyn[];
+    __shared__ int32_t big[ORD_T], nbig;
+    if (threadIdx.x == 0) nbig = 0;
+    __syncthreads();
+    const int64_t k = (int64_t)blockIdx.x * ORD_T + threadIdx.x;
+    const int32_t a = k < nkeys ? start[k] : 0, e = k < nkeys ? start[k + 1] : 0;
     if (e - a > SEG_THREAD) {
-        const int slot = atomicAdd(&big[0], 1);
-        big[1 + slot] = (int32_t)k;
-        return;
-    }
-    if (e - a <= SEG_REG) {
+        big[atomicAdd(&nbig, 1)] = (int32_t)k;
+    } else if (e - a > SEG_REG) {
+        for (int32_t p = a + 1; p < e; ++p) {  // insertion sort, ascending
+            const uint32_t v = perm[p];
+            int32_t q = p - 1;
+            while (q >= a && perm[q] > v) {
+                perm[q + 1] = perm[q];
+                --q;
+            }
+            perm[q + 1] = v;
+        }
+    } else if (e - a > 1) {
         // registers: each value's rank among the (distinct) segment values is
         // its position
         uint32_t v[SEG_REG];
@@ -177,37 +220,20 @@ __global__ __launch_bounds__(256) void k_fine_order(const int32_t* __restrict__ 
             for (int j = 0; j < SEG_REG; ++j) r += (v[j] < v[i]) ? 1 : 0;
             if (i < n) perm[a + r] = v[i];
         }
-        return;
     }
-    for (int32_t p = a + 1; p < e; ++p) {  // insertion sort, ascending
-        const uint32_t v = perm[p];
-        int32_t q = p - 1;
-        while (q >= a && perm[q] > v) {
-            perm[q + 1] = perm[q];
-            --q;
-        }
-        perm[q + 1] = v;
-    }
-}
-
-__global__ __launch_bounds__(1024) void k_fine_order_big(const int32_t* __restrict__ start,
-                                                         uint32_t* __restrict__ perm,
-                                                         const int32_t* __restrict__ big,
-                                                         uint32_t* __restrict__ tmp) {
-    extern __shared__ uint32_t sdyn[];
-    const int nbig = big[0];
-    for (int e = blockIdx.x; e < nbig; e += gridDim.x) {
-        const int32_t k = big[1 + e];
-        const int32_t a = start[k], L = start[k + 1] - a;
+    __syncthreads();
+    const int nb = nbig;
+    for (int q = 0; q < nb; ++q) {
+        const int32_t a = start[big[q]], L = start[big[q] + 1] - a;
         int n = 1;
         while (n < L) n <<= 1;
         // LDS when it fits, else the scratch region [2a, 2a + n) of tmp,
         // disjoint between segments because n < 2L
         uint32_t* s = n <= SEG_BIG ? sdyn : tmp + 2 * (int64_t)a;
-        for (int i = threadIdx.x; i < n; i += blockDim.x) s[i] = i < L ? perm[a + i] : 0xFFFFFFFFu;
+        for (int i = threadIdx.x; i < n; i += ORD_T) s[i] = i < L ? perm[a + i] : 0xFFFFFFFFu;
         __syncthreads();
         bitonic(s, n);
-        for (int i = threadIdx.x; i < L; i += blockDim.x) perm[a + i] = s[i];
+        for (int i = threadIdx.x; i < L; i += ORD_T) perm[a + i] = s[i];
         __syncthreads();
     }
 }
@@ -226,7 +252,7 @@ int launch_fine_sort(ereb_ctx* c, const PropsReq* props) {
     // the host reads it (check_flags)
     if (c->fcount_dirty && (rc = fill_i32(c, c->d_fcount, 0, nk))) return rc;
     // ranks live in the first M words of the oversize-segment scratch, which
-    // k_fine_order_big uses only after the placement
+    // k_fine_order uses only after the placement
     int32_t* rank = (int32_t*)c->d_tmp;
     if (M > 0) {
         c->fcount_dirty = true;
@@ -237,32 +263,16 @@ int launch_fine_sort(ereb_ctx* c, const PropsReq* props) {
         if (!props)
             hipLaunchKernelGGL(k_fine_count<NoProps>, dim3(nb), dim3(256), 0, c->stream, g,
                                c->nty, xm, ym, M, c->d_key, rank, c->d_fcount, c->d_flags,
-                               c->d_big, NoProps{});
+                               NoProps{});
         else {
-            // the key pass's completion as ev_keys when asked (rec_keys)
-            hipEvent_t done = c->rec_keys ? c->ev_keys : nullptr;
-            c->rec_keys = false;
-            if (marker_is_f32(c->precision, EREB_M_ETATOTALM)) {
-                const auto P = prop_args<float>(c, *props);
-                if (done)
-                    hipExtLaunchKernelGGL(k_fine_count<PropArgs<float>>, dim3(nb), dim3(256), 0,
-                                          c->stream, nullptr, done, 0, g, c->nty, xm, ym, M,
-                                          c->d_key, rank, c->d_fcount, c->d_flags, c->d_big, P);
-                else
-                    hipLaunchKernelGGL(k_fine_count<PropArgs<float>>, dim3(nb), dim3(256), 0,
-                                       c->stream, g, c->nty, xm, ym, M, c->d_key, rank,
-                                       c->d_fcount, c->d_flags, c->d_big, P);
-            } else {
-                const auto P = prop_args<double>(c, *props);
-                if (done)
-                    hipExtLaunchKernelGGL(k_fine_count<PropArgs<double>>, dim3(nb), dim3(256),
-                                          0, c->stream, nullptr, done, 0, g, c->nty, xm, ym, M,
-                                          c->d_key, rank, c->d_fcount, c->d_flags, c->d_big, P);
-                else
-                    hipLaunchKernelGGL(k_fine_count<PropArgs<double>>, dim3(nb), dim3(256), 0,
-                                       c->stream, g, c->nty, xm, ym, M, c->d_key, rank,
-                                       c->d_fcount, c->d_flags, c->d_big, P);
-            }
+            auto keys = [&](auto kern, auto P) {
+                hipLaunchKernelGGL(kern, dim3(nb), dim3(256), 0, c->stream, g, c->nty, xm, ym, M,
+                                   c->d_key, rank, c->d_fcount, c->d_flags, P);
+            };
+            if (marker_is_f32(c->precision, EREB_M_ETATOTALM))
+                keys(k_fine_count<PropArgs<float>>, prop_args<float>(c, *props));
+            else
+                keys(k_fine_count<PropArgs<double>>, prop_args<double>(c, *props));
         }
         if (props && c->scal_ride) {  // the device block now follows this launch
             c->scal_ride = false;
@@ -274,14 +284,19 @@ int launch_fine_sort(ereb_ctx* c, const PropsReq* props) {
     if ((rc = scan_exclusive(c, c->d_fcount, c->d_fstart, nk, nullptr, true))) return rc;
     c->fcount_dirty = false;
     if (M > 0) {
-        const unsigned nkb = (unsigned)((nk + 255) / 256);
         const unsigned nb = (unsigned)((M + 255) / 256);
-        hipLaunchKernelGGL(k_fine_place, dim3(nb), dim3(256), 0, c->stream, c->d_key,
-                           (const int32_t*)rank, M, c->d_fstart, c->d_perm);
-        hipLaunchKernelGGL(k_fine_order, dim3(nkb), dim3(256), 0, c->stream, c->d_fstart, nk,
-                           c->d_perm, c->d_big);
-        hipLaunchKernelGGL(k_fine_order_big, dim3(64), dim3(1024), SEG_BIG * sizeof(uint32_t),
-                           c->stream, c->d_fstart, c->d_perm, c->d_big, c->d_tmp);
+        if (c->tables_ride) {
+            const unsigned nt = rk4_coef_blocks(c);
+            hipLaunchKernelGGL(k_fine_place_tables, dim3(nb + 4 * nt), dim3(256), 0, c->stream,
+                               c->d_key, (const int32_t*)rank, M, c->d_fstart, c->d_perm, nb, nt,
+                               rk4_coef_args(c));
+            c->tables_ride = false;
+        } else
+            hipLaunchKernelGGL(k_fine_place, dim3(nb), dim3(256), 0, c->stream, c->d_key,
+                               (const int32_t*)rank, M, c->d_fstart, c->d_perm);
+        hipLaunchKernelGGL(k_fine_order, dim3((unsigned)((nk + ORD_T - 1) / ORD_T)), dim3(ORD_T),
+                           SEG_BIG * sizeof(uint32_t), c->stream, c->d_fstart, nk, c->d_perm,
+                           c->d_tmp);
     }
     EREB_HIP(c, hipGetLastError());
     prof_end(c, EREB_K_SORT, ev);
