@@ -24,7 +24,7 @@ def test_key_counts(Nx, Ny, crowd):
     M = 20_011
     x, y = g.xsize * rng.random(M), g.ysize * rng.random(M)
     for c in range(crowd and 30):  # 30 crowded quarter cells, some of them neighbours
-        k = slice(c * crowd // 2, c * crowd // 2 + crowd)
+        k = slice(c * crowd, (c + 1) * crowd)
         x[k] = 50.0 * (c % (2 * (Nx - 1))) + 5 + 40 * rng.random(x[k].size)
         y[k] = 50.0 * (c % (2 * (Ny - 1))) + 5 + 40 * rng.random(x[k].size)
     p = rng.permutation(M)
