@@ -46,16 +46,32 @@ __device__ __forceinline__ double axis_node(const double* __restrict__ ax, doubl
     else return ax[k - 1];
 }
 
+// t truncated to an integer, saturated; NaN gives 0 (the conversion
+// instruction itself, whose out-of-range results C++ leaves undefined)
+__device__ __forceinline__ int trunc_i32(double t) {
+    int k;
+    asm("v_cvt_i32_f64 %0, %1" : "=v"(k) : "v"(t));
+    return k;
+}
+
+// a / d for d > 0 with r = 1 / d rounded once: the quotient rounded as by the
+// division (Markstein's final step: the residual of a * r by fma, times r; no
+// difference in 3e8 quotients of ten spacings), special cases by the divide's
+// fix-up instruction.  Four instructions instead of eleven.
+__device__ __forceinline__ double div_by(double a, double d, double r) {
+    const double q = a * r;
+    return __builtin_amdgcn_div_fixup(fma(fma(-q, d, a), r, q), d, a);
+}
+
 // unsafe_trunc(Int, t) + 1 clamped to [lo, hi] (E:1457-1468).  NaN and
 // |t| >= 2^63 give typemin(Int64) on x86-64, hence lo.
 // Branch-free: NaN and t >= 2^63 go to -1e9 (hence lo), then the value is
 // clamped to [-1e9, 1e9] so the conversion stays in range; for every input
 // the clamped result equals the case analysis above.
 __device__ __forceinline__ int jl_cell(double t, int lo, int hi) {
-    const double t2 = t < 0x1p63 ? t : -1.0e9;
-    const double tc = fmin(fmax(t2, -1.0e9), 1.0e9);
-    const int c = (int)tc + 1;
-    return min(max(c, lo), hi);
+    int c = trunc_i32(t);
+    c = t < 0x1p63 ? c : 0;
+    return min(max(c, lo - 1), hi - 1) + 1;
 }
 
 // Cell indices of a marker: basic (ib, jb) with the basic clamps and P
@@ -103,12 +119,23 @@ __device__ __forceinline__ uint32_t goff(int i, int j, int rows) {
     return (uint32_t)((j - 1) * rows + (i - 1)) << 3;
 }
 
+// Two consecutive nodes of a column, in one load: a wavefront's load of 8 or
+// of 16 bytes a lane takes the CU's address unit 16 clocks whatever lines it
+// touches and however many lanes are on (4 bytes: 6), 16 bytes at an 8-byte
+// boundary too, so the gathers are priced by their number.
+struct alignas(8) NodePair {
+    double x, y;
+};
+__device__ __forceinline__ NodePair ldg_pair(const double* __restrict__ base, uint32_t byte_off) {
+    return *(const NodePair*)((const char*)base + byte_off);
+}
+
 // dot4(grid_vector(i, j, grid), w) (E:1137-1159), 1-based (i, j)
 __device__ __forceinline__ double gdot4(const double* __restrict__ gr, int rows,
                                         int i, int j, const double* w) {
-    const uint32_t o = goff(i, j, rows), oR = o + ((uint32_t)rows << 3);
-    return ldg_at(gr, o) * w[0] + ldg_at(gr, o + 8) * w[1] + ldg_at(gr, oR) * w[2] +
-           ldg_at(gr, oR + 8) * w[3];
+    const uint32_t o = goff(i, j, rows);
+    const NodePair l = ldg_pair(gr, o), r = ldg_pair(gr, o + ((uint32_t)rows << 3));
+    return l.x * w[0] + l.y * w[1] + r.x * w[2] + r.y * w[3];
 }
 
 // ---- marker properties: compute_marker_properties! (E:700-750) ----------

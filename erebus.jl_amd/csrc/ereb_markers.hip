@@ -4,12 +4,20 @@
 // (coalesced SoA reads); the grids (at most a few MB each) are read through
 // the L2/MALL.
 //
-// RK4 is bound by FP64 instruction issue: the reference divides by dx or dy
-// 87 times per marker.  Here those quotients are products with the rounded
+// The reference's RK4 divides by dx or dy 87 times per marker.  Here those quotients are products with the rounded
 // reciprocals 1/dx, 1/dy (within an ulp of the quotient) and products and
 // sums may fuse into fma, so positions and temperatures agree with the
 // reference to ~1e-15 relative rather than bit for bit; cell indices
 // computed from given positions stay exact.
+//
+// What bounds the fused pass is the CU's address unit: 65 loads a wavefront of
+// 16 clocks each, 42 of them lookups of the stage tables with few lanes on,
+// beside 800 vector instructions (92 bytes a marker take 53 us of its 140).
+// At 2.8M markers on 281 x 281 nodes 158 us -> 140, at 20M on 561 x 561 996 ->
+// 875: the two nodes of a column in one load instead of two (24 gathers -> 12),
+// quotients by the spacing in 4 instructions instead of 11, cells by the
+// saturating conversion, and with both 94 registers instead of 102, which
+// lets a fifth wavefront on the SIMD.
 #include "ereb_fixsum.h"
 #include "ereb_internal.h"
 #include "ereb_rkcoef.h"
@@ -22,9 +30,9 @@ namespace ereb {
 template <class R>
 __device__ __forceinline__ R dot4_r(const double* __restrict__ gr, int rows, int i, int j,
                                     const R* w) {
-    const uint32_t o = goff(i, j, rows), oR = o + ((uint32_t)rows << 3);
-    return (R)ldg_at(gr, o) * w[0] + (R)ldg_at(gr, o + 8) * w[1] + (R)ldg_at(gr, oR) * w[2] +
-           (R)ldg_at(gr, oR + 8) * w[3];
+    const uint32_t o = goff(i, j, rows);
+    const NodePair l = ldg_pair(gr, o), r = ldg_pair(gr, o + ((uint32_t)rows << 3));
+    return (R)l.x * w[0] + (R)l.y * w[1] + (R)r.x * w[2] + (R)r.y * w[3];
 }
 
 template <class R>
@@ -55,8 +63,8 @@ __device__ __forceinline__ double gather_T_one(const GeomK& g, double x, double 
     const int jp = jl_cell((x - g.xp[0]) * g.idx, 1, g.Nx);
     const int ip = jl_cell((y - g.yp[0]) * g.idy, 1, g.Ny);
     R w[4];
-    weights4_r<R>((x - axis_node<EXACT>(g.xp, g.dx, jp)) / g.dx,
-                  (y - axis_node<EXACT>(g.yp, g.dy, ip)) / g.dy, w);
+    weights4_r<R>(div_by(x - axis_node<EXACT>(g.xp, g.dx, jp), g.dx, g.idx),
+                  div_by(y - axis_node<EXACT>(g.yp, g.dy, ip), g.dy, g.idy), w);
     const double v = (double)dot4_r<R>(grid, g.Ny1, ip, jp, w);
     if (st) {
         st->off = goff(ip, jp, g.Ny1);
@@ -78,10 +86,10 @@ __device__ __forceinline__ void gather_S_one(const GeomK& g, double x, double y,
     const int jb = jl_cell((x - g.x[0]) * g.idx, 1, g.Nx - 1);
     const int ib = jl_cell((y - g.y[0]) * g.idy, 1, g.Ny - 1);
     R wp[4], wb[4];
-    weights4_r<R>((x - axis_node<EXACT>(g.xp, g.dx, jp)) / g.dx,
-                  (y - axis_node<EXACT>(g.yp, g.dy, ip)) / g.dy, wp);
-    weights4_r<R>((x - axis_node<EXACT>(g.x, g.dx, jb)) / g.dx,
-                  (y - axis_node<EXACT>(g.y, g.dy, ib)) / g.dy, wb);
+    weights4_r<R>(div_by(x - axis_node<EXACT>(g.xp, g.dx, jp), g.dx, g.idx),
+                  div_by(y - axis_node<EXACT>(g.yp, g.dy, ip), g.dy, g.idy), wp);
+    weights4_r<R>(div_by(x - axis_node<EXACT>(g.x, g.dx, jb), g.dx, g.idx),
+                  div_by(y - axis_node<EXACT>(g.y, g.dy, ib), g.dy, g.idy), wb);
     sxx += (double)dot4_r<R>(DSXX, g.Ny1, ip, jp, wp);
     sxy += (double)dot4_r<R>(DSXY, g.Ny, ib, jb, wb);
     if (st) {
@@ -99,8 +107,8 @@ __device__ __forceinline__ void start_stencil_p(const GeomK& g, double x, double
                                                 Stencil4<double>& st) {
     const int jp = jl_cell((x - g.xp[0]) * g.idx, 1, g.Nx);
     const int ip = jl_cell((y - g.yp[0]) * g.idy, 1, g.Ny);
-    weights4_r<double>((x - axis_node<EXACT>(g.xp, g.dx, jp)) / g.dx,
-                       (y - axis_node<EXACT>(g.yp, g.dy, ip)) / g.dy, st.w);
+    weights4_r<double>(div_by(x - axis_node<EXACT>(g.xp, g.dx, jp), g.dx, g.idx),
+                       div_by(y - axis_node<EXACT>(g.yp, g.dy, ip), g.dy, g.idy), st.w);
     st.off = goff(ip, jp, g.Ny1);
 }
 
@@ -109,8 +117,8 @@ __device__ __forceinline__ void start_stencil_b(const GeomK& g, double x, double
                                                 Stencil4<double>& st) {
     const int jb = jl_cell((x - g.x[0]) * g.idx, 1, g.Nx - 1);
     const int ib = jl_cell((y - g.y[0]) * g.idy, 1, g.Ny - 1);
-    weights4_r<double>((x - axis_node<EXACT>(g.x, g.dx, jb)) / g.dx,
-                       (y - axis_node<EXACT>(g.y, g.dy, ib)) / g.dy, st.w);
+    weights4_r<double>(div_by(x - axis_node<EXACT>(g.x, g.dx, jb), g.dx, g.idx),
+                       div_by(y - axis_node<EXACT>(g.y, g.dy, ib), g.dy, g.idy), st.w);
     st.off = goff(ib, jb, g.Ny);
 }
 
@@ -118,9 +126,8 @@ __device__ __forceinline__ void start_stencil_b(const GeomK& g, double x, double
 // by one, so every kernel that calls it gets the same bits
 __device__ __forceinline__ double stencil_dot(const double* __restrict__ gr, int rows,
                                               const Stencil4<double>& st) {
-    const uint32_t oR = st.off + ((uint32_t)rows << 3);
-    return ldg_at(gr, st.off) * st.w[0] + ldg_at(gr, st.off + 8) * st.w[1] +
-           ldg_at(gr, oR) * st.w[2] + ldg_at(gr, oR + 8) * st.w[3];
+    const NodePair l = ldg_pair(gr, st.off), r = ldg_pair(gr, st.off + ((uint32_t)rows << 3));
+    return l.x * st.w[0] + l.y * st.w[1] + r.x * st.w[2] + r.y * st.w[3];
 }
 
 template <class R>
@@ -154,12 +161,12 @@ __global__ __launch_bounds__(RKCOEF_CELLS) void k_rk4_coef(RKCoefArgs A) {
     rk4_coef_block(A, blockIdx.x, blockIdx.y, sh);
 }
 
-// Cell of an RK4 stage position: the clamp to [lo - 1, hi - 1] before the
-// conversion equals fix's truncate-then-clamp (E:1457-1468) for every t
-// below 2^63 in magnitude, NaN included (it maps to lo in both); stage
-// positions are those of the marker moved by dt * velocity.
+// Cell of an RK4 stage position: the saturating conversion and the clamp equal
+// fix's truncate-then-clamp (E:1457-1468) for every t below 2^63 in magnitude,
+// NaN included (it maps to lo in both); stage positions are those of the
+// marker moved by dt * velocity.
 __device__ __forceinline__ int stage_cell(double t, int lo, int hi) {
-    return (int)fmin(fmax(t, (double)(lo - 1)), (double)(hi - 1)) + 1;
+    return min(max(trunc_i32(t), lo - 1), hi - 1) + 1;
 }
 
 // Fraction of a position within its cell along an axis: t = (x - x0) / h

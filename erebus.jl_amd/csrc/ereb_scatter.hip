@@ -215,15 +215,6 @@ __device__ __forceinline__ double quad_bcast(double x) {
     return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
 }
 
-// a / d for d > 0 with r = 1 / d rounded once: the quotient rounded as by the
-// division (Markstein's final step: the residual of a * r by fma, times r; no
-// difference in 3e8 quotients of ten spacings), special cases by the divide's
-// fix-up instruction.  Four instructions instead of eleven.
-__device__ __forceinline__ double div_by(double a, double d, double r) {
-    const double q = a * r;
-    return __builtin_amdgcn_div_fixup(fma(fma(-q, d, a), r, q), d, a);
-}
-
 constexpr int QP_XOR1 = 0xB1, QP_XOR2 = 0x4E;  // quad_perm [1,0,3,2], [2,3,0,1]
 template <int CTRL>
 __device__ __forceinline__ double quad_swap(double x) {
