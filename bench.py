@@ -55,8 +55,8 @@ from ereb import precision, synth  # noqa: E402
 
 METRIC = "marker-steps/s, 2.8M markers: FP64 vs mixed-precision; adjoint/forward ratio"
 # how ereb_step_transfer issues a step (the library's default)
-STEP_LAUNCHES = ("eager on two streams: gathers + RK4 beside the node pass and assemblies "
-                 "once the scatter is done (graph replay off)")
+STEP_LAUNCHES = ("eager; above 400,000 markers on two streams: gathers + RK4 beside the node "
+                 "pass and assemblies once the scatter is done (graph replay off)")
 HBM_PEAK_GBS = 8000.0
 START_TIME = 2.25e6 * 365.25 * 24 * 3600  # C:339
 
@@ -93,11 +93,11 @@ STEP_CLASSES = ["sort", "scatter", "combine", "nodes", "rk4", "asm_sd", "asm_t"]
 # traffic summary (profiles/hbm_traffic_<workload>.json, made by
 # erebus.jl_amd/ereb/rocprof_summary.py from FETCH_SIZE / WRITE_SIZE runs)
 TRAFFIC_KERNEL = {
-    "fp64": {"scatter": "void ereb::k_scatter<double>", "rk4": "void ereb::k_rk4<1, true>",
+    "fp64": {"scatter": "void ereb::k_scatter<double,", "rk4": "void ereb::k_rk4<1, true>",
              "sort": "void ereb::k_fine_count<ereb::PropArgs<double>",
              "nodes": "ereb::k_combine_nodes", "asm_sd": "void ereb::k_asm_rows<0>",
              "asm_t": "void ereb::k_asm_rows<1>"},
-    "mixed": {"scatter": "void ereb::k_scatter<float>", "rk4": "void ereb::k_rk4<2, true>",
+    "mixed": {"scatter": "void ereb::k_scatter<float,", "rk4": "void ereb::k_rk4<2, true>",
               "sort": "void ereb::k_fine_count<ereb::PropArgs<float>",
               "nodes": "ereb::k_combine_nodes", "asm_sd": "void ereb::k_asm_rows<0>",
               "asm_t": "void ereb::k_asm_rows<1>"},
