@@ -639,9 +639,9 @@ struct OnStream {
 // the step writes, and write marker state that the sort and the scatter read;
 // the node pass and the two assemblies read the scatter's window sums and
 // node grids only.  So the marker pass (SEG_MARKERS) runs on the second
-// stream as soon as the scatter (SEG_SCATTER, whose sort also fills the
-// marker pass's coefficient tables) is done, beside the node pass and the
-// assemblies (SEG_NODES); the main stream waits for the second at the end.
+// stream, after its coefficient tables, as soon as the scatter (SEG_SCATTER)
+// is done, beside the node pass and the assemblies (SEG_NODES); the main stream
+// waits for the second at the end.
 // Results are those of the launches in sequence: no kernel of one stream
 // touches what the other's write.
 enum { SEG_SCATTER = 0, SEG_MARKERS, SEG_NODES };
@@ -654,18 +654,23 @@ enum { SEG_SCATTER = 0, SEG_MARKERS, SEG_NODES };
 // 43 / 90, 45 / 85, 77 / 108, 172 / 199.
 constexpr int64_t ONE_STREAM_MAX = 400000;
 
+// the marker pass's coefficient tables filled beside the sort's placement, not
+// before the marker pass (per-launch timing keeps them with its class)
+static bool tables_with_sort(const ereb_ctx* c) {
+    return c->marknum > 0 && c->marknum <= ONE_STREAM_MAX && !c->prof;
+}
+
 static int seg_launches(ereb_ctx* c, int seg, const double* hrs, const double* hrf,
                         int64_t mode, double dt, int64_t timestep) {
     int rc;
     switch (seg) {
         case SEG_SCATTER:
-            c->tables_ride = c->marknum > 0 && !c->prof;
+            c->tables_ride = tables_with_sort(c);
             rc = launch_scatter(c, hrs, hrf, (int)mode);
             c->tables_ride = false;
             return rc;
         case SEG_MARKERS:
-            // timed per class: the tables with the marker pass, else beside the sort
-            return launch_gathers_rk4(c, dt, (int)mode, timestep, c->prof);
+            return launch_gathers_rk4(c, dt, (int)mode, timestep, !tables_with_sort(c));
         default:
             if ((rc = launch_combine_nodes(c))) return rc;
             return launch_assemble_both(c, dt);

@@ -19,7 +19,7 @@
 //                     (in the transfer step also the RK4 coefficient tables,
 //                     by workgroups of their own);
 //   4. k_fine_order : each key segment (about 9 markers) is sorted by marker
-//                     index in place (in registers up to 16 markers),
+//                     index in place (in registers up to 32 markers),
 //                     removing the arrival order of step 3;
 //                     segments longer than SEG_THREAD by the whole workgroup
 //                     (bitonic in LDS up to 16384, global memory beyond).
@@ -156,9 +156,10 @@ __global__ __launch_bounds__(256) void k_fine_place(const uint32_t* __restrict__
 // The placement and, in the workgroups from nplace on, the RK4 coefficient
 // tables, which depend on the velocities only: in a launch of their own on the
 // second stream they cost the step a launch and two event calls (~15 us of
-// host time; the step of a 15 x 15 grid is its launches), and take the
-// placement's memory latency here (16 us alone, 18 with the tables at 2.8M
-// markers).
+// host time; the step of a 15 x 15 grid is its launches).  Only in the steps
+// that run on one stream: the tables' writes slow the placement down (35 us
+// together at 2.8M markers, where they take 14 and 12 apart; 203 at 20M, 77 and
+// 35), and beside the node pass and the assemblies they cost nothing.
 __global__ __launch_bounds__(256) void k_fine_place_tables(const uint32_t* __restrict__ key,
                                                            const int32_t* __restrict__ rank,
                                                            int64_t M,
@@ -177,14 +178,50 @@ __global__ __launch_bounds__(256) void k_fine_place_tables(const uint32_t* __res
     rk4_coef_block(A, (int)(b % ntab), (int)(b / ntab), sh);
 }
 
-constexpr int SEG_REG = 16;     // segments ordered in registers by rank
+constexpr int SEG_REG = 32;     // segments ordered in registers
 constexpr int SEG_THREAD = 48;  // longest segment ordered by one thread
 constexpr int SEG_BIG = 16384;  // longest segment ordered in LDS (64 KB)
 constexpr int ORD_T = 1024;     // keys per workgroup
 
+// Bitonic sorting network on N registers, ascending (Batcher 1968; every merge
+// begins with the flip, so all comparators point the same way): 80 comparators
+// of a minimum and a maximum for 16 values, 240 for 32.
+template <int N, int K, bool FLIP>
+__device__ __forceinline__ void net_stage(uint32_t (&v)[N]) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const int l = FLIP ? i ^ (K - 1) : i ^ K;
+        if (l > i) {
+            const uint32_t lo = min(v[i], v[l]), hi = max(v[i], v[l]);
+            v[i] = lo;
+            v[l] = hi;
+        }
+    }
+    if constexpr (FLIP ? K > 2 : K > 1) net_stage<N, FLIP ? K / 4 : K / 2, false>(v);
+}
+template <int N, int K = 2>
+__device__ __forceinline__ void net_sort(uint32_t (&v)[N]) {
+    net_stage<N, K, true>(v);
+    if constexpr (K < N) net_sort<N, 2 * K>(v);
+}
+template <int N>
+__device__ __forceinline__ void order_regs(uint32_t* __restrict__ seg, int n) {
+    uint32_t v[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] = i < n ? seg[i] : 0xffffffffu;
+    net_sort<N>(v);
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+        if (i < n) seg[i] = v[i];
+}
+
 // one thread per key; keys of more than SEG_THREAD markers are then ordered by
 // the whole workgroup, one after the other (a launch of its own for them, with
 // nothing to do in most steps, cost 5 us).  tmp: scratch of 2 M words.
+// What bounds it: the keys' dependent memory accesses and, with many markers a
+// key, a workgroup's longest one.  Up to 32 markers the network (before: ranks
+// up to 16, 16 n^2 comparisons, then insertion in memory): at 20M markers, 16 a
+// key on average, the sort 700 us -> 572, at 2.8M, 9 a key, 98 -> 96.
 __global__ __launch_bounds__(ORD_T) void k_fine_order(const int32_t* __restrict__ start,
                                                       int64_t nkeys, uint32_t* __restrict__ perm,
                                                       uint32_t* __restrict__ tmp) {
@@ -206,20 +243,10 @@ __global__ __launch_bounds__(ORD_T) void k_fine_order(const int32_t* __restrict_
             }
             perm[q + 1] = v;
         }
+    } else if (e - a > SEG_REG / 2) {
+        order_regs<SEG_REG>(perm + a, e - a);
     } else if (e - a > 1) {
-        // registers: each value's rank among the (distinct) segment values is
-        // its position
-        uint32_t v[SEG_REG];
-        const int n = e - a;
-#pragma unroll
-        for (int i = 0; i < SEG_REG; ++i) v[i] = i < n ? perm[a + i] : 0xffffffffu;
-#pragma unroll
-        for (int i = 0; i < SEG_REG; ++i) {
-            int r = 0;
-#pragma unroll
-            for (int j = 0; j < SEG_REG; ++j) r += (v[j] < v[i]) ? 1 : 0;
-            if (i < n) perm[a + r] = v[i];
-        }
+        order_regs<SEG_REG / 2>(perm + a, e - a);
     }
     __syncthreads();
     const int nb = nbig;

@@ -41,3 +41,28 @@ def test_key_counts(Nx, Ny, crowd):
             perm, key, nkeys = ctx.sort_order()
             assert np.array_equal(key, key_o)
             assert np.array_equal(perm, perm_o)
+
+
+def test_segment_lengths():
+    """Quarter cells of 1 to 50 markers each: the register networks of 16 and 32
+    (padded), insertion to 48, the workgroup beyond."""
+    g = Geometry(Nx=26, Ny=7, xsize=2500.0, ysize=600.0)
+    mat = Materials(marker_property_mode=1)
+    rng = np.random.default_rng(3)
+    n = np.tile(np.arange(1, 51), 12)  # 50 x 12 quarter cells of 50 m
+    q = np.repeat(np.arange(n.size), n)
+    p = rng.permutation(q.size)
+    q = q[p]
+    x = 50.0 * (q % 50) + 5 + 40 * rng.random(q.size)
+    y = 50.0 * (q // 50) + 5 + 40 * rng.random(q.size)
+    perm_o, key_o, _ = Oracle(g, mat).fine_sort(x, y)
+    lengths = np.bincount(np.asarray(key_o, dtype=np.int64))
+    assert set(range(1, 51)) <= set(lengths[lengths > 0].tolist())
+    one = np.ones(x.size)
+    with ereb.Context(g, mat, ereb.FP64) as ctx:
+        ctx.set_markers({"xm": x, "ym": y, "tm": np.full(x.size, 1), "tkm": 200 * one,
+                         "phim": 0.1 * one})
+        ctx.step_scatter(np.zeros(3), np.zeros(3), 1)
+        perm, key, _ = ctx.sort_order()
+    assert np.array_equal(key, key_o)
+    assert np.array_equal(perm, perm_o)
