@@ -248,9 +248,9 @@ static int reserve(ereb_ctx* c, int64_t n) {
     uint32_t *key = nullptr, *perm = nullptr, *tmp = nullptr;
     hipError_t e = hipMalloc(&key, sizeof(uint32_t) * n);
     if (e == hipSuccess) e = hipMalloc(&perm, sizeof(uint32_t) * n);
-    // oversize tile segments are sorted in [2*start, 2*start + pow2(len)),
-    // disjoint between tiles and inside [0, 2n)
-    if (e == hipSuccess) e = hipMalloc(&tmp, sizeof(uint32_t) * 2 * n);
+    // the longest key segments are sorted in [2*start, 2*start + pow2(len)),
+    // disjoint between keys and inside [0, 2n); the list of their keys follows
+    if (e == hipSuccess) e = hipMalloc(&tmp, sizeof(uint32_t) * (2 * n + sort_list_words(n)));
     if (e != hipSuccess) {
         hipFree(key);
         hipFree(perm);
@@ -262,7 +262,6 @@ static int reserve(ereb_ctx* c, int64_t n) {
     c->d_key = key;
     c->d_perm = perm;
     c->d_tmp = tmp;
-    c->tmp_cap = 2 * n;
     c->cap = n;
     c->have_sort = false;
     ++c->pos_gen;

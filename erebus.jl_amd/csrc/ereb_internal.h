@@ -140,8 +140,8 @@ struct ereb_ctx {
     int64_t nkeys = 0;             // ntiles * NFINE
     uint32_t* d_key = nullptr;     // cap
     uint32_t* d_perm = nullptr;    // cap
-    uint32_t* d_tmp = nullptr;     // 2*cap scratch: the sort's ranks, then oversize key segments
-    int64_t tmp_cap = 0;
+    uint32_t* d_tmp = nullptr;     // 2*cap scratch: the sort's ranks, then its longest key segments;
+                                   // after it the list of those keys (sort_list)
     int32_t* d_fcount = nullptr;   // nkeys
     int32_t* d_fstart = nullptr;   // nkeys + 1
     int32_t* d_flags = nullptr;    // [0] domain error
@@ -240,20 +240,25 @@ int prof_collect(ereb_ctx* c);
 
 // ---- kernel launchers ---------------------------------------------------
 // ereb_scan.hip: exclusive scan of n int32 into out[0..n], out[n] = total;
-// optionally a copy of out[0..n) in out2 and in[] zeroed once read
-// optionally only when run[0] != 0 (a device-side condition)
+// optionally the indices of inputs above `limit` appended to `above` (above[0]
+// counts them; zero before), in[] zeroed once read, only when run[0] != 0 (a
+// device-side condition)
 int scan_exclusive(ereb_ctx* c, const int32_t* in, int32_t* out, int64_t n,
-                   int32_t* out2 = nullptr, bool zero_in = false,
+                   int32_t* above = nullptr, int32_t limit = 0, bool zero_in = false,
                    const int32_t* run = nullptr);
 // the same with a caller-provided block-sum buffer of scan_blocks(n) ints
 int64_t scan_blocks(int64_t n);
 int scan_exclusive_buf(ereb_ctx* c, const int32_t* in, int32_t* out, int64_t n,
-                       int32_t* blocksums, int32_t* out2 = nullptr, bool zero_in = false,
-                       const int32_t* run = nullptr);
+                       int32_t* blocksums, int32_t* above = nullptr, int32_t limit = 0,
+                       bool zero_in = false, const int32_t* run = nullptr);
 // fill kernel (graph-safe replacement for hipMemsetAsync)
 int fill_i32(ereb_ctx* c, int32_t* p, int32_t v, int64_t n);
 int fill_f64(ereb_ctx* c, double* p, double v, int64_t n);
 
+// ereb_sort.hip: the key segments of more than SEG_WAVE markers, at most one
+// per SEG_WAVE + 1 markers of the capacity: their number, then their keys
+constexpr int SEG_WAVE = 1024;
+inline int64_t sort_list_words(int64_t cap) { return cap / (SEG_WAVE + 1) + 2; }
 // ereb_sort.hip: stable counting sort of marker indices by fine key; with
 // props, the pass that computes the keys also evaluates the marker
 // properties (compute_marker_properties!) with these heating rates and mode

@@ -59,12 +59,14 @@ __global__ __launch_bounds__(SCAN_T) void k_scan_blocksum(const int32_t* __restr
 
 // out[i] = exclusive prefix of in, the block's offset being the sum of the
 // block sums before it (each block adds them up itself); the last block also
-// writes the total to out[n].  Optionally also out2[i] = out[i], and in[i] = 0
-// once read (for inputs that must start from zero next time).
+// writes the total to out[n].  Optionally also in[i] = 0 once read (for inputs
+// that must start from zero next time), and the indices i of inputs above
+// `limit` appended to `above` in any order (above[0] counts them).
 __global__ __launch_bounds__(SCAN_T) void k_scan_apply(int32_t* __restrict__ in, int64_t n,
                                                        const int32_t* __restrict__ bs,
                                                        int32_t* __restrict__ out,
-                                                       int32_t* __restrict__ out2, int zero_in,
+                                                       int32_t* __restrict__ above,
+                                                       int32_t limit, int zero_in,
                                                        const int32_t* __restrict__ run) {
     __shared__ int32_t sh[SCAN_T / 64 + 1];
     if (run && run[0] == 0) return;
@@ -89,7 +91,7 @@ __global__ __launch_bounds__(SCAN_T) void k_scan_apply(int32_t* __restrict__ in,
     for (int k = 0; k < SCAN_PER; ++k) {
         if (base + k < n) {
             out[base + k] = e;
-            if (out2) out2[base + k] = e;
+            if (above && v[k] > limit) above[1 + atomicAdd(&above[0], 1)] = (int32_t)(base + k);
             if (zero_in) in[base + k] = 0;
         }
         e += v[k];
@@ -103,7 +105,8 @@ __global__ __launch_bounds__(SCAN_T) void k_scan_apply(int32_t* __restrict__ in,
 constexpr int64_t SCAN_ONE = 4 * SCAN_B;
 __global__ __launch_bounds__(SCAN_T) void k_scan_one(int32_t* __restrict__ in, int64_t n,
                                                      int32_t* __restrict__ out,
-                                                     int32_t* __restrict__ out2, int zero_in,
+                                                     int32_t* __restrict__ above,
+                                                     int32_t limit, int zero_in,
                                                      const int32_t* __restrict__ run) {
     __shared__ int32_t sh[SCAN_T / 64 + 1];
     if (run && run[0] == 0) return;
@@ -121,7 +124,7 @@ __global__ __launch_bounds__(SCAN_T) void k_scan_one(int32_t* __restrict__ in, i
         for (int k = 0; k < SCAN_PER; ++k) {
             if (base + k < n) {
                 out[base + k] = e;
-                if (out2) out2[base + k] = e;
+                if (above && v[k] > limit) above[1 + atomicAdd(&above[0], 1)] = (int32_t)(base + k);
                 if (zero_in) in[base + k] = 0;
             }
             e += v[k];
@@ -134,10 +137,11 @@ __global__ __launch_bounds__(SCAN_T) void k_scan_one(int32_t* __restrict__ in, i
 int64_t scan_blocks(int64_t n) { return std::max<int64_t>((n + SCAN_B - 1) / SCAN_B, 1); }
 
 int scan_exclusive_buf(ereb_ctx* c, const int32_t* in, int32_t* out, int64_t n,
-                       int32_t* blocksums, int32_t* out2, bool zero_in, const int32_t* run) {
+                       int32_t* blocksums, int32_t* above, int32_t limit, bool zero_in,
+                       const int32_t* run) {
     if (n <= SCAN_ONE) {
         hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(SCAN_T), 0, c->stream,
-                           const_cast<int32_t*>(in), n, out, out2, zero_in ? 1 : 0, run);
+                           const_cast<int32_t*>(in), n, out, above, limit, zero_in ? 1 : 0, run);
         EREB_HIP(c, hipGetLastError());
         return EREB_OK;
     }
@@ -145,17 +149,17 @@ int scan_exclusive_buf(ereb_ctx* c, const int32_t* in, int32_t* out, int64_t n,
     hipLaunchKernelGGL(k_scan_blocksum, dim3((unsigned)nb), dim3(SCAN_T), 0, c->stream, in, n,
                        blocksums, run);
     hipLaunchKernelGGL(k_scan_apply, dim3((unsigned)nb), dim3(SCAN_T), 0, c->stream,
-                       const_cast<int32_t*>(in), n, (const int32_t*)blocksums, out, out2,
-                       zero_in ? 1 : 0, run);
+                       const_cast<int32_t*>(in), n, (const int32_t*)blocksums, out, above,
+                       limit, zero_in ? 1 : 0, run);
     EREB_HIP(c, hipGetLastError());
     return EREB_OK;
 }
 
-int scan_exclusive(ereb_ctx* c, const int32_t* in, int32_t* out, int64_t n, int32_t* out2,
-                   bool zero_in, const int32_t* run) {
+int scan_exclusive(ereb_ctx* c, const int32_t* in, int32_t* out, int64_t n, int32_t* above,
+                   int32_t limit, bool zero_in, const int32_t* run) {
     int rc = ensure_scan(c, n);
     if (rc) return rc;
-    return scan_exclusive_buf(c, in, out, n, c->d_scan, out2, zero_in, run);
+    return scan_exclusive_buf(c, in, out, n, c->d_scan, above, limit, zero_in, run);
 }
 
 template <typename T>

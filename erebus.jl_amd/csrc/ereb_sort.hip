@@ -19,10 +19,13 @@
 //                     (in the transfer step also the RK4 coefficient tables,
 //                     by workgroups of their own);
 //   4. k_fine_order : each key segment (about 9 markers) is sorted by marker
-//                     index in place (in registers up to 32 markers),
-//                     removing the arrival order of step 3;
-//                     segments longer than SEG_THREAD by the whole workgroup
-//                     (bitonic in LDS up to 16384, global memory beyond).
+//                     index in place, removing the arrival order of step 3: up
+//                     to 32 markers by a thread in registers, up to 1,024 by a
+//                     wavefront in registers, the longer ones (listed by step 2)
+//                     by a workgroup each (bitonic in LDS up to 16384, global
+//                     memory beyond).
+#include <algorithm>
+
 #include "ereb_internal.h"
 #include "ereb_rkcoef.h"
 
@@ -95,9 +98,11 @@ __global__ __launch_bounds__(256) void k_fine_count(GeomK g, int nty, const doub
                                                     uint32_t* __restrict__ key,
                                                     int32_t* __restrict__ rank,
                                                     int32_t* __restrict__ count,
-                                                    int32_t* __restrict__ flags, P props) {
+                                                    int32_t* __restrict__ flags,
+                                                    int32_t* __restrict__ big, P props) {
     const int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const bool active = m < M;
+    if (m == 0) big[0] = 0;  // the scan, which lists the longest segments, runs after
     uint32_t k = 0;
     if (active) {
         bool bad;
@@ -178,10 +183,11 @@ __global__ __launch_bounds__(256) void k_fine_place_tables(const uint32_t* __res
     rk4_coef_block(A, (int)(b % ntab), (int)(b / ntab), sh);
 }
 
-constexpr int SEG_REG = 32;     // segments ordered in registers
-constexpr int SEG_THREAD = 48;  // longest segment ordered by one thread
+constexpr int SEG_REG = 32;     // longest segment ordered by one thread, in registers
+static_assert(SEG_WAVE == 16 * 64, "16 registers a lane");  // longest of one wavefront
 constexpr int SEG_BIG = 16384;  // longest segment ordered in LDS (64 KB)
-constexpr int ORD_T = 1024;     // keys per workgroup
+constexpr int ORD_T = 1024;     // threads of a workgroup, and its most keys
+constexpr int ORD_MIN = 16;     // its fewest keys: one a wavefront
 
 // Bitonic sorting network on N registers, ascending (Batcher 1968; every merge
 // begins with the flip, so all comparators point the same way): 80 comparators
@@ -215,43 +221,92 @@ __device__ __forceinline__ void order_regs(uint32_t* __restrict__ seg, int n) {
         if (i < n) seg[i] = v[i];
 }
 
-// one thread per key; keys of more than SEG_THREAD markers are then ordered by
-// the whole workgroup, one after the other (a launch of its own for them, with
-// nothing to do in most steps, cost 5 us).  tmp: scratch of 2 M words.
-// What bounds it: the keys' dependent memory accesses and, with many markers a
-// key, a workgroup's longest one.  Up to 32 markers the network (before: ranks
-// up to 16, 16 n^2 comparisons, then insertion in memory): at 20M markers, 16 a
-// key on average, the sort 700 us -> 572, at 2.8M, 9 a key, 98 -> 96.
-__global__ __launch_bounds__(ORD_T) void k_fine_order(const int32_t* __restrict__ start,
-                                                      int64_t nkeys, uint32_t* __restrict__ perm,
-                                                      uint32_t* __restrict__ tmp) {
-    extern __shared__ uint32_t sdyn[];
-    __shared__ int32_t big[ORD_T], nbig;
-    if (threadIdx.x == 0) nbig = 0;
-    __syncthreads();
-    const int64_t k = (int64_t)blockIdx.x * ORD_T + threadIdx.x;
-    const int32_t a = k < nkeys ? start[k] : 0, e = k < nkeys ? start[k + 1] : 0;
-    if (e - a > SEG_THREAD) {
-        big[atomicAdd(&nbig, 1)] = (int32_t)k;
-    } else if (e - a > SEG_REG) {
-        for (int32_t p = a + 1; p < e; ++p) {  // insertion sort, ascending
-            const uint32_t v = perm[p];
-            int32_t q = p - 1;
-            while (q >= a && perm[q] > v) {
-                perm[q + 1] = perm[q];
-                --q;
-            }
-            perm[q + 1] = v;
+// The same network over a wavefront, E values a lane (value i in lane i / E):
+// each lane's values, then merges of 2, 4, .. 64 lanes, whose comparators
+// across lanes are shuffles
+template <int E>
+__device__ __forceinline__ void wave_sort(uint32_t (&v)[E], int lane) {
+    if constexpr (E > 1) net_sort<E>(v);
+#pragma unroll 1
+    for (int w = 2; w <= 64; w <<= 1) {
+        uint32_t o[E];
+        const bool up = lane & (w >> 1);  // this lane keeps the maxima
+#pragma unroll
+        for (int e = 0; e < E; ++e) o[e] = __shfl_xor(v[E - 1 - e], w - 1, 64);
+#pragma unroll
+        for (int e = 0; e < E; ++e) v[e] = up ? max(v[e], o[e]) : min(v[e], o[e]);
+#pragma unroll 1
+        for (int d = w >> 2; d > 0; d >>= 1) {
+            const bool u = lane & d;
+#pragma unroll
+            for (int e = 0; e < E; ++e) o[e] = __shfl_xor(v[e], d, 64);
+#pragma unroll
+            for (int e = 0; e < E; ++e) v[e] = u ? max(v[e], o[e]) : min(v[e], o[e]);
         }
-    } else if (e - a > SEG_REG / 2) {
-        order_regs<SEG_REG>(perm + a, e - a);
-    } else if (e - a > 1) {
-        order_regs<SEG_REG / 2>(perm + a, e - a);
+        if constexpr (E > 1) net_stage<E, E / 2, false>(v);
+    }
+}
+template <int E>
+__device__ __forceinline__ void order_wave(uint32_t* __restrict__ seg, int n, int lane) {
+    uint32_t v[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) v[e] = lane * E + e < n ? seg[lane * E + e] : 0xffffffffu;
+    wave_sort<E>(v, lane);
+#pragma unroll
+    for (int e = 0; e < E; ++e)
+        if (lane * E + e < n) seg[lane * E + e] = v[e];
+}
+
+// keys of a workgroup of the ordering pass: at most one a thread; fewer where
+// that leaves the 256 CUs without a workgroup each (a small grid's wavefronts
+// then share its crowded keys), and fewer the more markers a key holds, so that
+// a workgroup has about 16,384 markers
+static int order_keys(int64_t nkeys, int64_t M) {
+    const int64_t chip = nkeys / 256;
+    const int64_t load = (int64_t)SEG_BIG * nkeys / std::max<int64_t>(M, 1);
+    return (int)std::clamp<int64_t>(std::min(chip, load), ORD_MIN, ORD_T);
+}
+
+// One thread per key of the workgroup's nper; the longer segments are then
+// dealt to its wavefronts, and those of more than SEG_WAVE markers, listed in
+// big, to the workgroups of the launch (a launch of its own for them, with
+// nothing to do in most steps, cost 5 us).  tmp: scratch of 2 M words.
+// What bounds it: the keys' dependent memory accesses; 64 registers, so that a
+// CU holds two workgroups.  The sort with every key crowded (16 x 16 markers a
+// cell) took 3,072 us at 15 x 15 nodes and 4,408 at 141 x 141 with such segments
+// ordered one after another by the workgroup that holds their 1,024 keys; 18 and
+// 189 now.
+__global__ __launch_bounds__(ORD_T, 8) void k_fine_order(const int32_t* __restrict__ start,
+                                                         int64_t nkeys, int nper,
+                                                         uint32_t* __restrict__ perm,
+                                                         const int32_t* __restrict__ big,
+                                                         uint32_t* __restrict__ tmp) {
+    extern __shared__ uint32_t sdyn[];
+    __shared__ int32_t left[ORD_T], nleft;  // keys left to the wavefronts
+    if (threadIdx.x == 0) nleft = 0;
+    __syncthreads();
+    const int64_t k = (int64_t)blockIdx.x * nper + threadIdx.x;
+    const bool mine = (int)threadIdx.x < nper && k < nkeys;
+    const int32_t a = mine ? start[k] : 0, n = mine ? start[k + 1] - a : 0;
+    if (n > SEG_REG) {
+        if (n <= SEG_WAVE) left[atomicAdd(&nleft, 1)] = (int32_t)k;
+    } else if (n > SEG_REG / 2) {
+        order_regs<SEG_REG>(perm + a, n);
+    } else if (n > 1) {
+        order_regs<SEG_REG / 2>(perm + a, n);
     }
     __syncthreads();
-    const int nb = nbig;
-    for (int q = 0; q < nb; ++q) {
-        const int32_t a = start[big[q]], L = start[big[q] + 1] - a;
+    const int lane = threadIdx.x & 63;
+    for (int q = threadIdx.x >> 6; q < nleft; q += ORD_T / 64) {
+        const int32_t a = start[left[q]], n = start[left[q] + 1] - a;
+        if (n <= 64) order_wave<1>(perm + a, n, lane);
+        else if (n <= 128) order_wave<2>(perm + a, n, lane);
+        else if (n <= 256) order_wave<4>(perm + a, n, lane);
+        else if (n <= 512) order_wave<8>(perm + a, n, lane);
+        else order_wave<16>(perm + a, n, lane);
+    }
+    for (int q = blockIdx.x; q < big[0]; q += gridDim.x) {
+        const int32_t a = start[big[1 + q]], L = start[big[1 + q] + 1] - a;
         int n = 1;
         while (n < L) n <<= 1;
         // LDS when it fits, else the scratch region [2a, 2a + n) of tmp,
@@ -281,6 +336,7 @@ int launch_fine_sort(ereb_ctx* c, const PropsReq* props) {
     // ranks live in the first M words of the oversize-segment scratch, which
     // k_fine_order uses only after the placement
     int32_t* rank = (int32_t*)c->d_tmp;
+    int32_t* big = rank + 2 * c->cap;  // sort_list_words(cap) words
     if (M > 0) {
         c->fcount_dirty = true;
         const unsigned nb = (unsigned)((M + 255) / 256);
@@ -290,11 +346,11 @@ int launch_fine_sort(ereb_ctx* c, const PropsReq* props) {
         if (!props)
             hipLaunchKernelGGL(k_fine_count<NoProps>, dim3(nb), dim3(256), 0, c->stream, g,
                                c->nty, xm, ym, M, c->d_key, rank, c->d_fcount, c->d_flags,
-                               NoProps{});
+                               big, NoProps{});
         else {
             auto keys = [&](auto kern, auto P) {
                 hipLaunchKernelGGL(kern, dim3(nb), dim3(256), 0, c->stream, g, c->nty, xm, ym, M,
-                                   c->d_key, rank, c->d_fcount, c->d_flags, P);
+                                   c->d_key, rank, c->d_fcount, c->d_flags, big, P);
             };
             if (marker_is_f32(c->precision, EREB_M_ETATOTALM))
                 keys(k_fine_count<PropArgs<float>>, prop_args<float>(c, *props));
@@ -308,7 +364,7 @@ int launch_fine_sort(ereb_ctx* c, const PropsReq* props) {
         }
     }
     // key starts; the counts are cleared for the next sort
-    if ((rc = scan_exclusive(c, c->d_fcount, c->d_fstart, nk, nullptr, true))) return rc;
+    if ((rc = scan_exclusive(c, c->d_fcount, c->d_fstart, nk, big, SEG_WAVE, true))) return rc;
     c->fcount_dirty = false;
     if (M > 0) {
         const unsigned nb = (unsigned)((M + 255) / 256);
@@ -321,9 +377,10 @@ int launch_fine_sort(ereb_ctx* c, const PropsReq* props) {
         } else
             hipLaunchKernelGGL(k_fine_place, dim3(nb), dim3(256), 0, c->stream, c->d_key,
                                (const int32_t*)rank, M, c->d_fstart, c->d_perm);
-        hipLaunchKernelGGL(k_fine_order, dim3((unsigned)((nk + ORD_T - 1) / ORD_T)), dim3(ORD_T),
-                           SEG_BIG * sizeof(uint32_t), c->stream, c->d_fstart, nk, c->d_perm,
-                           c->d_tmp);
+        const int nper = order_keys(nk, M);
+        hipLaunchKernelGGL(k_fine_order, dim3((unsigned)((nk + nper - 1) / nper)), dim3(ORD_T),
+                           SEG_BIG * sizeof(uint32_t), c->stream, c->d_fstart, nk, nper,
+                           c->d_perm, (const int32_t*)big, c->d_tmp);
     }
     EREB_HIP(c, hipGetLastError());
     prof_end(c, EREB_K_SORT, ev);

@@ -1,8 +1,8 @@
 """The sort's key starts and segment order at the sizes where its launches
-change: up to 16,384 keys are scanned by one workgroup, more by several; a
-workgroup of the ordering pass holds 1,024 keys, of which those with more than
-48 markers are ordered by the whole workgroup.  Fine keys and sort order
-bit-exact with the oracle's stable counting sort."""
+change: up to 16,384 keys are scanned by one workgroup, more by several; a key's
+segment is ordered by a thread up to 32 markers, by a wavefront up to 1,024, by
+a workgroup beyond.  Fine keys and sort order bit-exact with the oracle's stable
+counting sort."""
 from __future__ import annotations
 
 import numpy as np
@@ -45,7 +45,7 @@ def test_key_counts(Nx, Ny, crowd):
 
 def test_segment_lengths():
     """Quarter cells of 1 to 50 markers each: the register networks of 16 and 32
-    (padded), insertion to 48, the workgroup beyond."""
+    (padded), a wavefront beyond."""
     g = Geometry(Nx=26, Ny=7, xsize=2500.0, ysize=600.0)
     mat = Materials(marker_property_mode=1)
     rng = np.random.default_rng(3)
@@ -66,3 +66,64 @@ def test_segment_lengths():
         perm, key, _ = ctx.sort_order()
     assert np.array_equal(key, key_o)
     assert np.array_equal(perm, perm_o)
+
+
+# values a lane of the wavefront's network: 1, 2, 4, 8, 16; beyond, a workgroup
+# in LDS, then in memory
+EDGES = [0, 1, 32, 33, 64, 65, 128, 129, 256, 257, 512, 513, 1023, 1024, 1025, 2048, 2049,
+         5000, 16_385]
+
+
+@pytest.mark.parametrize("Nx,Ny", [(7, 7), (26, 7), (679, 7)])
+def test_long_segments(Nx, Ny):
+    """Neighbouring quarter cells at the edges of the ordering pass's ways: one
+    tile (144 keys), five, and more keys than the one-workgroup scan takes with
+    one marker in some of the others."""
+    g = Geometry(Nx=Nx, Ny=Ny, xsize=100.0 * (Nx - 1), ysize=100.0 * (Ny - 1))
+    mat = Materials(marker_property_mode=1)
+    rng = np.random.default_rng(Nx)
+    nq = 4 * (Nx - 1) * (Ny - 1)
+    n = (rng.random(nq) < 0.3).astype(np.int64)
+    at = np.concatenate([np.arange(len(EDGES)), nq - 1 - np.arange(len(EDGES))])
+    n[at] = np.concatenate([EDGES, EDGES])
+    q = np.repeat(np.arange(nq), n)
+    q = q[rng.permutation(q.size)]
+    rows = 2 * (Ny - 1)
+    x = 50.0 * (q // rows) + 5 + 40 * rng.random(q.size)
+    y = 50.0 * (q % rows) + 5 + 40 * rng.random(q.size)
+    perm_o, key_o, _ = Oracle(g, mat).fine_sort(x, y)
+    lengths = np.bincount(np.asarray(key_o, dtype=np.int64))
+    assert set(EDGES[1:]) <= set(lengths.tolist())
+    one = np.ones(x.size)
+    with ereb.Context(g, mat, ereb.FP64) as ctx:
+        ctx.set_markers({"xm": x, "ym": y, "tm": np.full(x.size, 1), "tkm": 200 * one,
+                         "phim": 0.1 * one})
+        for _ in range(2):  # the second finds the list of the first
+            ctx.step_scatter(np.zeros(3), np.zeros(3), 1)
+            perm, key, _ = ctx.sort_order()
+            assert np.array_equal(key, key_o)
+            assert np.array_equal(perm, perm_o)
+
+
+def test_crowded_keys_share_the_chip():
+    """Sixteen times the markers in the same cells, 64 a key, cost the sort far
+    less than sixteen times as much: 15 x 15 nodes have 1,296 keys, and ordered
+    one after another by the workgroup that holds them they took 200 times as
+    long as at 4 a key (3,072 against 15 us; 18 now)."""
+    us = {}
+    for mc in (4, 16):
+        g = Geometry(Nx=15, Ny=15, xsize=14_000.0, ysize=14_000.0, Nxmc=mc, Nymc=mc)
+        mat = Materials(marker_property_mode=1)
+        mk = ereb.synth.make_markers(g, mat, seed=1)
+        with ereb.Context(g, mat, ereb.FP64) as ctx:
+            ctx.set_markers(mk)
+            ctx.step_scatter(np.zeros(3), np.zeros(3), 1)
+            best = np.inf
+            for _ in range(5):
+                ctx.profile(True)
+                ctx.profile_reset()
+                ctx.step_scatter(np.zeros(3), np.zeros(3), 1)
+                ms, n = ctx.profile_get("sort")
+                best = min(best, ms / n)
+            us[mc] = best * 1e3
+    assert us[16] < 16 * us[4], us
