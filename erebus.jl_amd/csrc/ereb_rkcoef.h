@@ -63,7 +63,10 @@ __device__ __forceinline__ void rk_half(double* __restrict__ out, double a0, dou
 constexpr int RKCOEF_CELLS = 256;
 
 // bx: block of RKCOEF_CELLS cells, t: table; sh: RKCOEF_CELLS * RKC doubles of LDS
-__device__ __forceinline__ void rk4_coef_block(const RKCoefArgs& A, int bx, int t,
+// (A by value: of a reference's four tables the compiler picks one through
+// scratch memory, 40 bytes a lane, a third more writes than the tables'; the
+// launch with the placement at 141 x 141 nodes took 8.6 us, 5.9 now)
+__device__ __forceinline__ void rk4_coef_block(RKCoefArgs A, int bx, int t,
                                                double* __restrict__ sh) {
     const int R = A.Ny + 1;
     const int N = R * (A.Nx + 1);
