@@ -62,7 +62,7 @@ __device__ __forceinline__ double interp_grad(const GeomK& g, const double* gr, 
 // Where the grid cotangents of one grid go.  PASS 0 keeps the largest
 // |contribution| of the lane (as bits, which order non-negative doubles), taken
 // over the workgroup before one atomic a grid; one atomic a contribution, all
-// to one address, took 2.9 ms for 40,000 markers' RK4 pullback, 76 us now.
+// to one address, took 2.9 ms for 40,000 markers' RK4 pullback, 62 us now.
 // PASS 1 adds to the workgroup's window of the grid in LDS (integer adds, so
 // the order does not matter) and straight to the grid outside it; the window's
 // touched nodes then take one atomic pair each.  The 172 contributions of a
@@ -243,8 +243,11 @@ __device__ __forceinline__ double vx_stage(const GeomK& g, const double* v, cons
             const double r0 = vbar * (1.0 - b) * h, r1 = vbar * b * h;
             F.add(i, jq0, r0);
             F.add(i, jq2, r0);
-            if (right) F.add(i, jc, -2.0 * r0);
-            else Fc.add(i, jc, -2.0 * r0);
+            // one of the two grids, by value: as branches the compiler merges
+            // them into one addition through a pointer, and every grid's
+            // state goes to scratch memory (496 bytes a lane, 76 us)
+            F.add(i, jc, right ? -2.0 * r0 : 0.0);
+            Fc.add(i, jc, right ? 0.0 : -2.0 * r0);
             F.add(i + 1, jq0, r1);
             F.add(i + 1, jq2, r1);
             F.add(i + 1, jc, -2.0 * r1);

@@ -56,7 +56,7 @@ def scratch():
     return out
 
 
-@pytest.mark.parametrize("kernel", ["k_rk4_coef", "k_fine_place_tables"])
+@pytest.mark.parametrize("kernel", ["k_rk4_coef", "k_fine_place_tables", "k_rk4_pullback"])
 def test_no_scratch(scratch, kernel):
     found = {k: v for k, v in scratch.items() if f"{len(kernel)}{kernel}" in k}
     assert found
