@@ -226,19 +226,26 @@ __device__ __forceinline__ double quad_swap(double x) {
     return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
 }
 
+template <int CTRL>
+__device__ __forceinline__ float quad_swap(float x) {
+    return __int_as_float(
+        __builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, true));
+}
+
 // r[f] at lane t of a quad -> r[g] at lane j: the old r[j] of lane g
-__device__ __forceinline__ void quad_transpose(double (&r)[4], bool odd, bool high) {
+template <class V>
+__device__ __forceinline__ void quad_transpose(V (&r)[4], bool odd, bool high) {
 #pragma unroll
     for (int f = 0; f < 4; f += 2) {
-        const double a = r[f], b = r[f + 1];
-        const double ax = quad_swap<QP_XOR1>(a), bx = quad_swap<QP_XOR1>(b);
+        const V a = r[f], b = r[f + 1];
+        const V ax = quad_swap<QP_XOR1>(a), bx = quad_swap<QP_XOR1>(b);
         r[f] = odd ? bx : a;
         r[f + 1] = odd ? b : ax;
     }
 #pragma unroll
     for (int f = 0; f < 2; ++f) {
-        const double a = r[f], b = r[f + 2];
-        const double ax = quad_swap<QP_XOR2>(a), bx = quad_swap<QP_XOR2>(b);
+        const V a = r[f], b = r[f + 2];
+        const V ax = quad_swap<QP_XOR2>(a), bx = quad_swap<QP_XOR2>(b);
         r[f] = high ? bx : a;
         r[f + 2] = high ? b : ax;
     }
@@ -253,7 +260,7 @@ template <class R, bool TYPED> struct ChunkData {
     int32_t fj;                                          // fine column, -1: no marker
 };
 
-// loads of the lane's marker m
+// loads of the lane's marker, without the material vectors of untyped markers
 template <class R, bool TYPED>
 __device__ __forceinline__ void load_marker(const ScatterArgs<R>& A, uint32_t mk, int fj,
                                             ChunkData<R, TYPED>& D) {
@@ -275,15 +282,19 @@ __device__ __forceinline__ void load_marker(const ScatterArgs<R>& A, uint32_t mk
     D.tkrhocp = A.tkrhocp[m];
     D.rhocptotal = A.rhocptotal[m];
     D.hrtotal = A.hrtotal[m];
-    if constexpr (!TYPED) {
-        D.tens = A.tens[m];
-        D.frict = A.frict[m];
-        D.invggg = A.invggg[m];
-        D.cohes = A.cohes[m];
-        D.rhof = A.rhof[m];
-        D.alphas = A.alphas[m];
-        D.alphaf = A.alphaf[m];
-    }
+}
+template <class R>
+__device__ __forceinline__ void load_material(const ScatterArgs<R>& A, uint32_t mk,
+                                              ChunkData<R, false>& D) {
+    if (D.fj < 0) return;
+    const size_t m = mk;
+    D.tens = A.tens[m];
+    D.frict = A.frict[m];
+    D.invggg = A.invggg[m];
+    D.cohes = A.cohes[m];
+    D.rhof = A.rhof[m];
+    D.alphas = A.alphas[m];
+    D.alphaf = A.alphaf[m];
 }
 
 // addresses of strip rb's results (ScatterLDS::addr)
@@ -539,6 +550,7 @@ __global__ __launch_bounds__(SCAT_NW * 64, scat_waves(sizeof(R) == 4, TYPED)) vo
     {
         const uint32_t m = marker(0, fjx);
         load_marker<R, TYPED>(A, m, fjx, D);
+        if constexpr (!TYPED) load_material<R>(A, m, D);
     }
     uint32_t mx = marker(4, fjx);
     for (int s0 = 0; s0 < pre[SEGC]; s0 += 4) {
@@ -552,31 +564,46 @@ __global__ __launch_bounds__(SCAT_NW * 64, scat_waves(sizeof(R) == 4, TYPED)) vo
         const double yb = L.ax[2][ci >> 1], yp = L.ax[3][(ci + 1) >> 1];
         double fxb = div_by(D.x - xb, dx, rdx), fxp = div_by(D.x - xp, dx, rdx);
         double fyb = div_by(D.y - yb, dy, rdy), fyp = div_by(D.y - yp, dy, rdy);
-        int tm = D.fj >= 0 ? min(max(D.tm, 1), 3) : 0;
+        int tm = 0;
+        if constexpr (TYPED) tm = D.fj >= 0 ? min(max(D.tm, 1), 3) : 0;
         // done here, before the loads below (as the transposes)
-        asm volatile("" : "+v"(fxb), "+v"(fxp), "+v"(fyb), "+v"(fyp), "+v"(tm));
+        asm volatile("" : "+v"(fxb), "+v"(fxp), "+v"(fyb), "+v"(fyp));
+        if constexpr (TYPED) asm volatile("" : "+v"(tm));
         double q[P::nquad][4];
+        R qt[2][4];  // T1, T2: in the vectors' type until a product takes them
         {
-            const double one = D.fj >= 0 ? 1.0 : 0.0;
-            const double raw[5][4] = {
-                {(double)D.etatotal, (double)D.etavp, D.sxy, TYPED ? 0.0 : one},
-                {(double)D.rhototal, (double)D.ktotal, (double)D.etafkphi, D.phi},
-                {D.sxx, (double)D.tkrhocp, (double)D.rhocptotal, (double)D.hrtotal},
-                {(double)D.tens, (double)D.frict, (double)D.invggg, (double)D.cohes},
-                {(double)D.rhof, (double)D.alphas, (double)D.alphaf, one}};
+            const R one = D.fj >= 0 ? R(1) : R(0);
+            // done here: the selects would otherwise move into the groups
+            // below and hold twice the registers until then
+            auto turn = [&](auto& r) {
+                quad_transpose(r, t & 1, t & 2);
 #pragma unroll
-            for (int u = 0; u < (TYPED ? 3 : 5); ++u) {
+                for (int f = 0; f < 4; ++f) asm volatile("" : "+v"(r[f]));
+            };
+            const double raw[3][4] = {
+                {(double)D.etatotal, (double)D.etavp, D.sxy, TYPED ? 0.0 : (double)one},
+                {(double)D.rhototal, (double)D.ktotal, (double)D.etafkphi, D.phi},
+                {D.sxx, (double)D.tkrhocp, (double)D.rhocptotal, (double)D.hrtotal}};
+#pragma unroll
+            for (int u = 0; u < 3; ++u) {
 #pragma unroll
                 for (int f = 0; f < 4; ++f) q[u][f] = raw[u][f];
-                quad_transpose(q[u], t & 1, t & 2);
-                // done here: the selects would otherwise move into the groups
-                // below and hold twice the registers until then
+                turn(q[u]);
+            }
+            if constexpr (!TYPED) {
+                const R rawt[2][4] = {{D.tens, D.frict, D.invggg, D.cohes},
+                                      {D.rhof, D.alphas, D.alphaf, one}};
 #pragma unroll
-                for (int f = 0; f < 4; ++f) asm volatile("" : "+v"(q[u][f]));
+                for (int u = 0; u < 2; ++u) {
+#pragma unroll
+                    for (int f = 0; f < 4; ++f) qt[u][f] = rawt[u][f];
+                    turn(qt[u]);
+                }
             }
         }
         __builtin_amdgcn_sched_barrier(0);
         load_marker<R, TYPED>(A, mx, fjx, D);
+        const uint32_t m1 = mx;
         mx = marker(s0 + 8, fjx);
         __builtin_amdgcn_sched_barrier(0);
         auto group = [&](auto gc) {
@@ -590,7 +617,12 @@ __global__ __launch_bounds__(SCAT_NW * 64, scat_waves(sizeof(R) == 4, TYPED)) vo
             const double wxb = lb ? 1.0 - axb : axb, wxp = lp ? 1.0 - axp : axp;
             const double wyb = ls ? 1.0 - ayb : ayb, wyp = ls ? 1.0 - ayp : ayp;
             const double w[4] = {wyb * wxb, wyp * wxb, wyb * wxp, wyp * wxp};
-            if constexpr (TYPED) q[I][g] = quad_bcast<g>(tm) == t + 1 ? 1.0 : 0.0;
+            if constexpr (TYPED) {
+                q[I][g] = quad_bcast<g>(tm) == t + 1 ? 1.0 : 0.0;
+            } else {
+                q[T1][g] = (double)qt[0][g];
+                q[T2][g] = (double)qt[1][g];
+            }
 #pragma unroll
             for (int e = 0; e < P::nacc; ++e)
                 acc[e] = __builtin_amdgcn_mfma_f64_4x4x4f64(w[P::GRID[e]], q[P::QUAD[e]][g],
@@ -598,6 +630,15 @@ __global__ __launch_bounds__(SCAT_NW * 64, scat_waves(sizeof(R) == 4, TYPED)) vo
             while (col < f1 && s0 + g + 1 == end) next_col();
         };
         group(std::integral_constant<int, 0>{});
+        if constexpr (!TYPED) {
+            // once the first group's registers are free: with all loads ahead
+            // of it the Float64 form spilled one of 128 (176 us at 2.8M
+            // markers, 163 so; two workgroups a CU need at most 128), the
+            // mixed form took 141, 134 with its float quads
+            __builtin_amdgcn_sched_barrier(0);
+            load_material<R>(A, m1, D);
+            __builtin_amdgcn_sched_barrier(0);
+        }
         group(std::integral_constant<int, 1>{});
         group(std::integral_constant<int, 2>{});
         group(std::integral_constant<int, 3>{});

@@ -56,7 +56,8 @@ def scratch():
     return out
 
 
-@pytest.mark.parametrize("kernel", ["k_rk4_coef", "k_fine_place_tables", "k_rk4_pullback"])
+@pytest.mark.parametrize("kernel", ["k_rk4_coef", "k_fine_place_tables", "k_rk4_pullback",
+                                    "k_scatter"])
 def test_no_scratch(scratch, kernel):
     found = {k: v for k, v in scratch.items() if f"{len(kernel)}{kernel}" in k}
     assert found
