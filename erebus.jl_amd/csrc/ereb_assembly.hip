@@ -789,7 +789,7 @@ static int sys_ready(ereb_ctx* c, AsmSys& K) {
 // assembly (a fresh system) it is raised here.
 static int sys_fresh(ereb_ctx* c, Sys& s) {
     const int rc = s.have_prev ? EREB_OK : fill_i32(c, s.chg, 1, 1);
-    s.have_prev = true;
+    if (!rc) s.have_prev = true;
     return rc;
 }
 
