@@ -127,9 +127,23 @@ def _cells(x, y, x0, y0, dx, dy, jmin, jmax, imin, imax):
     return i, j
 
 
+# the marker vectors that the scatter sums
+SCATTERED = ["etatotalm", "etavpm", "inv_gggtotalm", "sxym", "cohestotalm", "tenstotalm",
+             "fricttotalm", "rhototalm", "rhofluidcur", "ktotalm", "phim",
+             "etafluidcur_inv_kphim", "rhocptotalm", "alphasolidcur", "alphafluidcur", "hrtotalm",
+             "sxxm", "tkm_rhocptotalm"]
+
+
 def abs_sums(g: Geometry, mk: dict, props: dict) -> list:
     """Per node sum of |property * weight| for the 30 SUM grids (the scale
     against which a reordered floating-point sum is compared)."""
+    return node_sums(g, mk, props, absolute=True)
+
+
+def node_sums(g: Geometry, mk: dict, props: dict, absolute: bool = False) -> list:
+    """Per node sum of property * weight for the 30 SUM grids, of the values
+    given (props over mk); absolute: of |property * weight|."""
+    mag = np.abs if absolute else np.asarray
     a = g.axes()
     Nx, Ny = g.Nx, g.Ny
     x, y = mk["xm"], mk["ym"]
@@ -154,17 +168,16 @@ def abs_sums(g: Geometry, mk: dict, props: dict) -> list:
     for gname in ("basic", "vx", "vy", "p"):
         ax, ay, lim, shp = spec[gname]
         i, j = _cells(x, y, ax[0], ay[0], g.dx, g.dy, *lim)
-        A = np.abs((x - ax[j - 1]) / g.dx)
-        B = np.abs((y - ay[i - 1]) / g.dy)
-        # |weights| as a sparse (node x marker) matrix, 4 entries per marker
-        # (column-major node index), applied to all |property| columns at once
-        w = np.stack([np.abs(1 - B) * np.abs(1 - A), B * np.abs(1 - A), np.abs(1 - B) * A,
-                      B * A], axis=1)
+        A = (x - ax[j - 1]) / g.dx
+        B = (y - ay[i - 1]) / g.dy
+        # weights as a sparse (node x marker) matrix, 4 entries per marker
+        # (column-major node index), applied to all property columns at once
+        w = mag(np.stack([(1 - B) * (1 - A), B * (1 - A), (1 - B) * A, B * A], axis=1))
         node = np.stack([(j - 1 + dj) * shp[0] + (i - 1 + di)
                          for di, dj in ((0, 0), (1, 0), (0, 1), (1, 1))], axis=1)
         W = scipy.sparse.csc_matrix((w.ravel(), node.ravel(), np.arange(0, 4 * M + 1, 4)),
                                     shape=(shp[0] * shp[1], M))
-        P = np.stack([np.ones_like(x) if f is None else np.abs(allv[f])
+        P = np.stack([np.ones_like(x) if f is None else mag(allv[f])
                       for f in fields[gname]], axis=1)
         S = W @ P
         out.extend(S[:, k].reshape(shp, order="F") for k in range(P.shape[1]))

@@ -3,24 +3,23 @@
 Markers pile up where the flow converges; the code paths that only crowded
 cells reach are held to the bars of the uniform parity tests:
   - a fine cell of 20,000 markers: the sort orders it by a bitonic sort in
-    global memory (more than 16,384 markers), the scatter walks its column in
-    chunks of 256 staged markers, the P-grid scatter reads the tile's sort
-    order from memory (more than 4,096 markers in the tile);
+    global memory (more than 16,384 markers), the scatter walks it in 5,000
+    groups of four, the P-grid scatter reads the tile's sort order from memory
+    (more than 4,096 markers in the tile);
   - a fine cell of 3,000 markers (bitonic sort in LDS), one of 30 (ordered
-    by one thread), 400 markers spread over one basic column (a column split
-    into chunks across many fine cells);
+    by one thread), 400 markers spread over one basic column (fine cells of a
+    few markers above each other);
   - markers exactly on basic and P node lines, on the box edges and outside
     the box (the clamps of the cell index, C:66-101).
 Bars: fine keys, sort order and marker properties bit-exact; Float64 node
-sums within 1e-12 of the per-node sum of |terms|; mixed-form node sums within
-1e-6 of the field's largest sum of |terms| (max|error| <= 1e-6 max|terms|
-sums, per field): the normwise bar of the mixed form, max|error| / max|sum|,
-wherever the terms share a sign.  The random-sign stresses of 20,000 markers
-in one cell cancel, which the plain normwise bar does not allow for
-(SXXSUM's error is 1.8e-6 of its largest sum); a per-node bar does not fit
-the mixed form either, whose float stencil fractions carry an absolute
-error of ~6e-8, large against a node's own sum where it gets only small
-weights.  Melt composition and the thermochemical sums as in the uniform
+sums within 1e-12 of the per-node sum of |terms|.  The mixed form's weights and
+sums are Float64 too, its property vectors float: its node sums are held to the
+same bar against the sums of the property values it holds, and within 1e-6 of
+the field's largest sum of |terms| against the oracle (max|error| <= 1e-6
+max|terms| sums, per field: the normwise bar of the mixed form, max|error| /
+max|sum|, wherever the terms share a sign; the random-sign stresses of 20,000
+markers in one cell cancel, which the plain normwise bar does not allow for).
+Melt composition and the thermochemical sums as in the uniform
 tests.  No
 marker and a single marker run every step without error and give the
 oracle's sums.
@@ -149,6 +148,10 @@ def test_crowded_scatter_mixed_form(crowded):
         ctx.set_markers(mk)
         ctx.step_scatter(hrs, hrf, 1)
         got = [ctx.get_grid(n) for n in ereb.SUM_FIELDS]
+        held = {n: ctx.get_marker(n) for n in cases.SCATTERED}
+    for n, a, b, c in zip(ereb.SUM_FIELDS, got, cases.node_sums(g, mk, held),
+                          cases.abs_sums(g, mk, held)):
+        assert np.all(np.abs(a - b) <= 1e-12 * c), n
     absb = cases.abs_sums(g, mk, props_o)
     for n, a, b, c in zip(ereb.SUM_FIELDS, got, sums_o, absb):
         err = np.abs(a - b).max() / max(c.max(), 1e-300)

@@ -1,7 +1,6 @@
-"""Mixed-precision form (EREB_MIXED): FP32 marker properties, weights,
-interpolation and per-fine-cell sums with compensated FP32 per-node
-accumulation; Float64 marker state, node normalisation and matrix
-coefficients.
+"""Mixed-precision form (EREB_MIXED): FP32 marker properties and stress
+interpolation; Float64 marker state, scatter weights and sums, node
+normalisation and matrix coefficients.
 
 Bar: every nodal field (the 30 SUM grids and the 27 normalised node fields)
 and every marker property within 1e-6 of the Float64 result, normwise

@@ -3,9 +3,11 @@ group, a chunk of four groups or a tile ends: fine cells (quarters of a basic
 cell) of 0 to 65 markers side by side, grids whose cells fill no tile and whose
 tiles are one cell wide, type-derived and free material vectors.
 
-Bars, as for the other scatter tests: Float64 node sums within 1e-12 of the
-per-node sum of |terms| (the order of the sum differs), mixed form within 1e-6
-of the field's largest sum of |terms| (float property vectors)."""
+Bars: node sums within 1e-12 of the per-node sum of |terms| (the order of the
+sum differs), in the Float64 form against the oracle, in the mixed form against
+the sums of the property values it holds (its property vectors are float, its
+weights and sums Float64); those against the oracle within 1e-6 of the field's
+largest sum of |terms|."""
 from __future__ import annotations
 
 import numpy as np
@@ -64,6 +66,11 @@ def test_groups(Nx, Ny, typed, form):
         got = [ctx.get_grid(n) for n in ereb.SUM_FIELDS]
         ctx.step_scatter(hrs, hrf, 1)
         again = [ctx.get_grid(n) for n in ereb.SUM_FIELDS]
+        held = {n: ctx.get_marker(n) for n in cases.SCATTERED}
+    if form == ereb.MIXED:
+        own = cases.node_sums(g, mk, held)
+        for n, a, b, c in zip(ereb.SUM_FIELDS, got, own, cases.abs_sums(g, mk, held)):
+            assert np.all(np.abs(a - b) <= 1e-12 * c), n
     for n, a, b, c, d in zip(ereb.SUM_FIELDS, got, sums, scale, again):
         bar = 1e-12 * c if form == ereb.FP64 else 1e-6 * c.max()
         assert np.all(np.abs(a - b) <= bar), n
