@@ -235,10 +235,10 @@ int ereb_step_assemble_thermal(ereb_ctx* ctx, double dt, int64_t* nnz);
  * the node pass and the assemblies, which read none of the marker state it
  * writes; the call returns with the context's stream ordered after both.  With
  * graph replay on (ereb_ctx_set_graphs), after the first call the step's
- * launches are captured once into three graphs (of both streams) and replayed; they
- * are captured again when the mode, the marker count, the precision form or
- * a device buffer changes (not when dt, the heating rates or the timestep
- * change).  Results are those of the separate calls, bit for bit.  Every
+ * launches are captured once into three graphs and replayed, on both streams
+ * whatever the marker count; they are captured again when the mode, the marker
+ * count, the precision form or a device buffer changes (not when dt, the
+ * heating rates or the timestep change).  Results are those of the separate calls, bit for bit.  Every
  * launch in sequence on the context's stream while profiling is enabled. */
 int ereb_step_transfer(ereb_ctx* ctx, const double hrsolidm[3],
                        const double hrfluidm[3], int64_t mode, double dt,

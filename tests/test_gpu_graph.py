@@ -137,9 +137,9 @@ def test_graph_replay_across_replenishment():
 
 @pytest.mark.parametrize("M", [0, 1])
 def test_step_with_no_marker_and_one_marker(M):
-    """The two-stream step and its graph replays with 0 and 1 markers (the
-    marker branch then launches nothing, or one workgroup's worth): equal to
-    the separate resident calls bit for bit, step after step."""
+    """The step with 0 and 1 markers (the marker pass then launches nothing, or
+    one workgroup's worth), eager on one stream and as graph replays on two:
+    equal to the separate resident calls bit for bit, step after step."""
     g, mat = synth.workload_geometry("adj41", mode=1)
     mk = synth.make_markers(g, mat, seed=9)
     pick = np.arange(M) * 977 % mk["xm"].size
@@ -202,6 +202,60 @@ def test_two_stream_step_at_workload_size(precision):
             assert np.array_equal(sa[k], sc[k], equal_nan=True), k
             assert np.array_equal(sb[k], sc[k], equal_nan=True), k
         assert B.graph_stats()[1] == 3  # steps 2-4 replayed
+    finally:
+        A.close()
+        B.close()
+        C.close()
+
+
+def test_step_across_the_stream_rule():
+    """One context stepped with marker counts below, at and above the 400,000
+    up to which an eager step runs on one stream with its coefficient tables
+    filled beside the sort's placement; above, they are filled on the second
+    stream.  The velocities change from step to step, so that stale tables
+    would show.  Eager and with graph replay (two streams at every count),
+    equal to the separate resident calls bit for bit."""
+    g, mat = synth.workload_geometry("fp64", mode=1)
+    full = synth.make_markers(g, mat, seed=2, stress=True)
+    p = np.sort(np.random.default_rng(4).choice(full["xm"].size, 400_001, replace=False))
+    full = {k: np.ascontiguousarray(v[p]) for k, v in full.items()}
+    vx, vy = synth.stream_velocity(g)
+    A = _ctx(g, mat, full, graphs=False)
+    B = _ctx(g, mat, full, graphs=True)
+    C = _ctx(g, mat, full, graphs=False)
+    try:
+        ts = 0
+        for M in (400_001, 400_000, 399_999, 400_001):
+            mk = {k: v[:M] for k, v in full.items()}
+            for c in (A, B, C):
+                c.set_markers(mk)
+            for _ in range(3):
+                ts += 1
+                dt, hrs, hrf = _scalars(mat, ts)
+                f = 1.0 + 0.1 * np.sin(ts)
+                for c in (A, B, C):
+                    c.set_grid("vx", f * vx)
+                    c.set_grid("vy", f * vy)
+                    c.set_grid("vxf", (2.0 - f) * vx)
+                    c.set_grid("vyf", (2.0 - f) * vy)
+                for c in (A, B):
+                    c.step_transfer(hrs, hrf, 1, dt, ts)
+                C.step_scatter(hrs, hrf, 1)
+                C.step_node_properties()
+                C.step_assemble_stokes_darcy(dt)
+                C.step_assemble_thermal(dt)
+                C.step_gather_stress()
+                C.step_gather_temperature(ts)
+                C.step_advect_rk4(dt, 1)
+                for n in ("xm", "ym", "tkm", "sxxm", "sxym"):
+                    a, b, c_ = A.get_marker(n), B.get_marker(n), C.get_marker(n)
+                    assert np.array_equal(a, c_) and np.array_equal(b, c_), (ts, M, n)
+            assert A.marknum == M
+        sa, sb, sc = _state(A), _state(B), _state(C)
+        for k in sc:
+            assert np.array_equal(sa[k], sc[k], equal_nan=True), k
+            assert np.array_equal(sb[k], sc[k], equal_nan=True), k
+        assert B.graph_stats()[1] >= 6
     finally:
         A.close()
         B.close()
