@@ -647,10 +647,21 @@ enum { SEG_SCATTER = 0, SEG_MARKERS, SEG_NODES };
 
 // Steps of at most this many markers run in sequence on the main stream.  The
 // second stream's event calls cost the host ~43 us a step, as much as all of
-// its 12 launches, and the marker pass that it hides is short.  us per step, one
-// stream / two: a context by itself 73 / 88 at 3,136 markers, 101 / 104 at
-// 160,000, 131 / 128 at 313,600, 216 / 198 at 1,000,000; three contexts in turn
-// 43 / 90, 45 / 85, 77 / 108, 172 / 199.
+// its 12 launches, and the marker pass that it hides is short.
+// us per step (Float64; 577,920 markers on inexact axes):
+//   markers       a context by itself    three contexts in turn
+//                 one stream     two     one stream     two
+//       3,136             73      88             43      90
+//     313,600            128     126             73     113
+//     577,920            151     132             97     136
+//   1,000,000            203     190            163     192
+//   2,822,400            460     444            388     411
+//  20,070,400          2,388   2,363          2,317   2,315
+// (mixed form: 395 / 376 and 337 / 362 at 2.8M, 2,070 / 2,057 and 2,017 / 2,007
+// at 20M.)  Several contexts in turn fill the chip with each other's kernels and
+// are never better off with two streams; a context by itself is, by more than 2%
+// from somewhere above 313,600 markers on.  The line is drawn for the context by
+// itself, the ordinary program.
 constexpr int64_t ONE_STREAM_MAX = 400000;
 
 // the marker pass's coefficient tables filled beside the sort's placement, not

@@ -63,11 +63,11 @@ __device__ __forceinline__ double div_by(double a, double d, double r) {
     return __builtin_amdgcn_div_fixup(fma(fma(-q, d, a), r, q), d, a);
 }
 
-// unsafe_trunc(Int, t) + 1 clamped to [lo, hi] (E:1457-1468).  NaN and
-// |t| >= 2^63 give typemin(Int64) on x86-64, hence lo.
-// Branch-free: NaN and t >= 2^63 go to -1e9 (hence lo), then the value is
-// clamped to [-1e9, 1e9] so the conversion stays in range; for every input
-// the clamped result equals the case analysis above.
+// unsafe_trunc(Int, t) + 1 clamped to [lo, hi] (E:1457-1468), 1 <= lo, hi below
+// 2^31.  NaN and |t| >= 2^63 give typemin(Int64) on x86-64, hence lo.
+// Branch-free: the conversion saturates, so |t| beyond 2^31 clamps to hi or lo
+// as its truncation would; NaN converts to 0 and t >= 2^63 is replaced by 0,
+// at or below lo - 1, hence lo.
 __device__ __forceinline__ int jl_cell(double t, int lo, int hi) {
     int c = trunc_i32(t);
     c = t < 0x1p63 ? c : 0;

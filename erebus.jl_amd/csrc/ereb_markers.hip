@@ -4,20 +4,26 @@
 // (coalesced SoA reads); the grids (at most a few MB each) are read through
 // the L2/MALL.
 //
-// The reference's RK4 divides by dx or dy 87 times per marker.  Here those quotients are products with the rounded
-// reciprocals 1/dx, 1/dy (within an ulp of the quotient) and products and
-// sums may fuse into fma, so positions and temperatures agree with the
-// reference to ~1e-15 relative rather than bit for bit; cell indices
-// computed from given positions stay exact.
+// The reference's RK4 divides by dx or dy 87 times per marker.  Here those
+// quotients are products with the rounded reciprocals 1/dx, 1/dy (within an ulp
+// of the quotient) and products and sums may fuse into fma, so positions and
+// temperatures agree with the reference to ~1e-15 relative rather than bit for
+// bit; cell indices computed from given positions stay exact.
 //
-// What bounds the fused pass is the CU's address unit: 65 loads a wavefront of
-// 16 clocks each, 42 of them lookups of the stage tables with few lanes on,
-// beside 800 vector instructions (92 bytes a marker take 53 us of its 140).
-// At 2.8M markers on 281 x 281 nodes 158 us -> 140, at 20M on 561 x 561 996 ->
-// 875: the two nodes of a column in one load instead of two (24 gathers -> 12),
-// quotients by the spacing in 4 instructions instead of 11, cells by the
-// saturating conversion, and with both 94 registers instead of 102, which
-// lets a fifth wavefront on the SIMD.
+// What the fused pass spends: its 65 loads a wavefront take the CU's address
+// unit 16 clocks each, 42 of them lookups of the stage tables with few lanes on
+// (75 us of the 133-141, by box, that it takes for 2.8M markers on 281 x 281
+// nodes with the tables); its 92 bytes a marker take 53; the rest is the latency
+// of eight rounds of dependent lookups at five wavefronts a SIMD.
+// At 2.8M markers 158 us -> 140, at 20M on 561 x 561 nodes 996 -> 875: the two
+// nodes of a column in one load instead of two (24 gathers -> 12), quotients by
+// the spacing in 4 instructions instead of 11, cells by the saturating
+// conversion, and with both 94 registers instead of 102, which lets a fifth
+// wavefront on the SIMD.  That holds for exact axes; with loaded ones it is 98
+// registers and four.  The fifth takes the registers that the node pass and the
+// assemblies ran in beside it on the other stream (the overlap of a step of 20M
+// markers fell from 82 to 50 us), yet held to four the whole step is slower:
+// 444 us -> 448 at 2.8M, 2,363 -> 2,391 at 20M (mixed 376 -> 386, 2,057 -> 2,089).
 #include "ereb_fixsum.h"
 #include "ereb_internal.h"
 #include "ereb_rkcoef.h"
