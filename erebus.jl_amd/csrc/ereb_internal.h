@@ -240,8 +240,8 @@ int prof_collect(ereb_ctx* c);
 
 // ---- kernel launchers ---------------------------------------------------
 // ereb_scan.hip: exclusive scan of n int32 into out[0..n], out[n] = total;
-// optionally the indices of inputs above `limit` appended to `above` (above[0]
-// counts them; zero before), in[] zeroed once read, only when run[0] != 0 (a
+// optionally the indices of inputs above `limit` listed from above[1] on in any
+// order, above[0] of them, in[] zeroed once read, only when run[0] != 0 (a
 // device-side condition)
 int scan_exclusive(ereb_ctx* c, const int32_t* in, int32_t* out, int64_t n,
                    int32_t* above = nullptr, int32_t limit = 0, bool zero_in = false,

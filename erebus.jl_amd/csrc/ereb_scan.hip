@@ -39,11 +39,13 @@ __device__ __forceinline__ int32_t block_exclusive_scan(int32_t v, int32_t* sh, 
     return r;
 }
 
-// sum of each block's SCAN_B inputs
+// sum of each block's SCAN_B inputs; above (optional): its count zeroed for
+// k_scan_apply
 // run (optional): the scan runs only when run[0] != 0 (a device-side
 // condition, so that a captured graph can skip it)
 __global__ __launch_bounds__(SCAN_T) void k_scan_blocksum(const int32_t* __restrict__ in,
                                                           int64_t n, int32_t* __restrict__ bs,
+                                                          int32_t* __restrict__ above,
                                                           const int32_t* __restrict__ run) {
     __shared__ int32_t sh[SCAN_T / 64 + 1];
     if (run && run[0] == 0) return;
@@ -55,6 +57,7 @@ __global__ __launch_bounds__(SCAN_T) void k_scan_blocksum(const int32_t* __restr
     int32_t tot;
     block_exclusive_scan(s, sh, &tot);
     if (threadIdx.x == 0) bs[blockIdx.x] = tot;
+    if (above && blockIdx.x == 0 && threadIdx.x == 0) above[0] = 0;
 }
 
 // out[i] = exclusive prefix of in, the block's offset being the sum of the
@@ -110,6 +113,8 @@ __global__ __launch_bounds__(SCAN_T) void k_scan_one(int32_t* __restrict__ in, i
                                                      const int32_t* __restrict__ run) {
     __shared__ int32_t sh[SCAN_T / 64 + 1];
     if (run && run[0] == 0) return;
+    // before the first of the scans below, whose barriers order it
+    if (above && threadIdx.x == 0) above[0] = 0;
     int32_t off = 0;
     for (int64_t b = 0; b < n; b += SCAN_B) {
         const int64_t base = b + (int64_t)threadIdx.x * SCAN_PER;
@@ -147,7 +152,7 @@ int scan_exclusive_buf(ereb_ctx* c, const int32_t* in, int32_t* out, int64_t n,
     }
     const int64_t nb = scan_blocks(n);
     hipLaunchKernelGGL(k_scan_blocksum, dim3((unsigned)nb), dim3(SCAN_T), 0, c->stream, in, n,
-                       blocksums, run);
+                       blocksums, above, run);
     hipLaunchKernelGGL(k_scan_apply, dim3((unsigned)nb), dim3(SCAN_T), 0, c->stream,
                        const_cast<int32_t*>(in), n, (const int32_t*)blocksums, out, above,
                        limit, zero_in ? 1 : 0, run);

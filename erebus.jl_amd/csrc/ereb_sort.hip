@@ -98,11 +98,9 @@ __global__ __launch_bounds__(256) void k_fine_count(GeomK g, int nty, const doub
                                                     uint32_t* __restrict__ key,
                                                     int32_t* __restrict__ rank,
                                                     int32_t* __restrict__ count,
-                                                    int32_t* __restrict__ flags,
-                                                    int32_t* __restrict__ big, P props) {
+                                                    int32_t* __restrict__ flags, P props) {
     const int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const bool active = m < M;
-    if (m == 0) big[0] = 0;  // the scan, which lists the longest segments, runs after
     uint32_t k = 0;
     if (active) {
         bool bad;
@@ -346,11 +344,11 @@ int launch_fine_sort(ereb_ctx* c, const PropsReq* props) {
         if (!props)
             hipLaunchKernelGGL(k_fine_count<NoProps>, dim3(nb), dim3(256), 0, c->stream, g,
                                c->nty, xm, ym, M, c->d_key, rank, c->d_fcount, c->d_flags,
-                               big, NoProps{});
+                               NoProps{});
         else {
             auto keys = [&](auto kern, auto P) {
                 hipLaunchKernelGGL(kern, dim3(nb), dim3(256), 0, c->stream, g, c->nty, xm, ym, M,
-                                   c->d_key, rank, c->d_fcount, c->d_flags, big, P);
+                                   c->d_key, rank, c->d_fcount, c->d_flags, P);
             };
             if (marker_is_f32(c->precision, EREB_M_ETATOTALM))
                 keys(k_fine_count<PropArgs<float>>, prop_args<float>(c, *props));
