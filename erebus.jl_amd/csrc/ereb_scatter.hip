@@ -565,10 +565,13 @@ __global__ __launch_bounds__(SCAT_NW * 64, scat_waves(sizeof(R) == 4, TYPED)) vo
         double fxb = div_by(D.x - xb, dx, rdx), fxp = div_by(D.x - xp, dx, rdx);
         double fyb = div_by(D.y - yb, dy, rdy), fyp = div_by(D.y - yp, dy, rdy);
         int tm = 0;
-        if constexpr (TYPED) tm = D.fj >= 0 ? min(max(D.tm, 1), 3) : 0;
         // done here, before the loads below (as the transposes)
-        asm volatile("" : "+v"(fxb), "+v"(fxp), "+v"(fyb), "+v"(fyp));
-        if constexpr (TYPED) asm volatile("" : "+v"(tm));
+        if constexpr (TYPED) {
+            tm = D.fj >= 0 ? min(max(D.tm, 1), 3) : 0;
+            asm volatile("" : "+v"(fxb), "+v"(fxp), "+v"(fyb), "+v"(fyp), "+v"(tm));
+        } else {
+            asm volatile("" : "+v"(fxb), "+v"(fxp), "+v"(fyb), "+v"(fyp));
+        }
         double q[P::nquad][4];
         R qt[2][4];  // T1, T2: in the vectors' type until a product takes them
         {
