@@ -672,7 +672,7 @@ def main():
         domm, roofsm, steproofm = rooflines(g, M, kernm, "mixed", a.workload, nnzm, msm)
         res["mixed"] = {
             "value": vm, "ms_per_step": msm, "speedup_vs_fp64": vm / value,
-            "dtype": "f32 properties/weights/interpolation, f64 state/normalisation/coefficients",
+            "dtype": "f32 properties/stress interpolation, f64 state/weights/sums/normalisation/coefficients",
             "roofline": dict(roofsm[domm], kernel_class=domm), "rooflines": roofsm,
             "step_roofline": steproofm, "launches": STEP_LAUNCHES,
             "kernel_ms": kernm,
