@@ -12,7 +12,7 @@
 //
 // What the fused pass spends: its 65 loads a wavefront take the CU's address
 // unit 16 clocks each, 42 of them lookups of the stage tables with few lanes on
-// (75 us of the 133-141, by box, that it takes for 2.8M markers on 281 x 281
+// (75 us of the 133-141, by machine, that it takes for 2.8M markers on 281 x 281
 // nodes with the tables); its 92 bytes a marker take 53; the rest is the latency
 // of eight rounds of dependent lookups at five wavefronts a SIMD.
 // At 2.8M markers 158 us -> 140, at 20M on 561 x 561 nodes 996 -> 875: the two
